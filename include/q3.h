@@ -78,7 +78,8 @@ int q3_gemv_partials(int M, int N, int epi);
  * SWIGLU}.  Replaces F.linear / cuBLAS in the prompt pass and at decode batches
  * above 64 (engine.py:439,450,803).  With q3_gemm_tiles_wide(M, N) the
  * 256 x 256-tile kernel (eight waves, direct global-to-LDS loads) runs, else
- * 16..128-row tiles.  K % 64 == 0; N % 4 == 0; ldx >= K, ldx % 8 == 0;
+ * one that streams the weights into MFMA operands beside loader waves for the
+ * tokens (tiles of 16..128 tokens x 32..256 weight rows).  K % 64 == 0; N % 4 == 0; ldx >= K, ldx % 8 == 0;
  * ldy % 4 == 0 (SWIGLU writes N/2 columns); x, W 16-byte and y 8-byte
  * aligned. */
 int q3_gemm(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
@@ -99,9 +100,11 @@ int q3_gemm_partials(const uint16_t *x, int ldx, const uint16_t *w, int M, int N
  * full -- or, at 256+ tokens below q3_gemm_tiles_wide, where all the tiles
  * fill at most half the CUs -- those tiles are split along K and a second
  * kernel sums their FP32 partials in split order and applies the epilogue;
- * the other tiles are q3_gemm's, bit for bit.  ws holds q3_gemm_ws_floats(M, N, K) floats
- * (0: no split tail, and q3_gemm_ws is q3_gemm), 16-byte aligned.  Same
- * operand rules as q3_gemm. */
+ * the other tiles are q3_gemm's, bit for bit.  Below 256 tokens, projections
+ * of long K may split K over all tiles the same way.  ws holds
+ * q3_gemm_ws_floats(M, N, K) floats (0: nothing is split, and q3_gemm_ws is
+ * q3_gemm), 16-byte aligned; up to 512 tokens it may be more than is used.
+ * Same operand rules as q3_gemm. */
 int q3_gemm_ws_floats(int M, int N, int K);
 int q3_gemm_ws(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
                int epi, uint16_t *y, int ldy, float *ws, hipStream_t stream);

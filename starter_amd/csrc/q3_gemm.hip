@@ -35,8 +35,9 @@
 //   to ws [splits, M, N], summed in split order by the consumer
 //   (add_rmsnorm_partials, which also applies the next RMSNorm).
 //
-// * narrow (few tiles: small prompts and decode batches above 64): 256
-//   threads, BM x BN tiles of up to 128 x 128, LDS staged through registers.
+// * mid (few tiles: short prompts and decode batches above 64): weights
+//   straight into MFMA operands, token rows through LDS by loader waves
+//   (q3_gemm_mid.hpp).
 //
 // Operands: A = W rows (n), B = x rows (m), so a lane's four C values are four
 // consecutive output columns of one token row (both halves of a SwiGLU pair in
@@ -44,36 +45,13 @@
 // where the output rows allow it (store_row16).
 #include "q3_common.hpp"
 #include "q3_dma.hpp"
+#include "q3_gemm_mid.hpp"
 #include "q3.h"
 
 namespace {
 
 using namespace q3dma;
-
-__device__ __forceinline__ f32x4_t mfma(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
-                                                   c, 0, 0, 0);
-}
-
-// Four consecutive output columns col..col+3 of token row m (col % 4 == 0).
-template <int EPI>
-__device__ __forceinline__ void store4(bf16_t* y, int ldy, int m, int col, const f32x4_t& v) {
-    if constexpr (EPI == Q3_EPI_SWIGLU) {
-        const uint32_t a = pack_bf16x2(v[0], v[1]), b = pack_bf16x2(v[2], v[3]);  // gate, up rounded
-        *reinterpret_cast<uint32_t*>(y + (int64_t)m * ldy + (col >> 1)) =
-            pack_bf16x2(silu_bf16(bflo(a)) * bfhi(a), silu_bf16(bflo(b)) * bfhi(b));
-    } else {
-        uint2* p = reinterpret_cast<uint2*>(y + (int64_t)m * ldy + col);
-        if constexpr (EPI == Q3_EPI_RESID) {
-            const uint2 r = *p;
-            const uint32_t a = pack_bf16x2(v[0], v[1]), b = pack_bf16x2(v[2], v[3]);
-            *p = make_uint2(pack_bf16x2(bflo(r.x) + bflo(a), bfhi(r.x) + bfhi(a)),
-                            pack_bf16x2(bflo(r.y) + bflo(b), bfhi(r.y) + bfhi(b)));
-        } else {
-            *p = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-        }
-    }
-}
+using namespace q3gemm;
 
 // ------------------------------------------------------------------ wide
 
@@ -143,12 +121,6 @@ constexpr int WIDE_CPR = 8;                          // 16-byte chunks per 128-b
 constexpr int WIDE_TCH = 256 * WIDE_CPR;             // chunks per operand tile
 constexpr int WIDE_DPT = WIDE_TCH / WIDE_THREADS;    // direct loads per operand per thread per step
 constexpr int WIDE_GROUP = 4;                        // token tiles per raster group
-constexpr int EPI_PARTIAL = -1;                      // FP32 split partials, no rounding
-
-// Position of 16-byte chunk c of 128-byte row r: c ^ ((r >> 1) & 7).  Measured
-// on gfx950: a ds_read_b128 whose 64 lanes read rows r0..r0+15 at one logical
-// chunk (four k groups) runs at the linear-read rate; no swizzle is 2.5x slower.
-__device__ __forceinline__ int wide_swz(int r) { return (r >> 1) & 7; }
 
 // Origin of tile t of a tm x tn grid in raster order: groups of WIDE_GROUP
 // token tiles sweeping the weight tiles (the group's token tiles share each
@@ -362,137 +334,6 @@ __global__ __launch_bounds__(256) void wide_tail_reduce_kernel(const float* __re
     store4<EPI>(y, ldy, m0 + r, n0 + c, a);
 }
 
-// ---------------------------------------------------------------- narrow
-
-constexpr int THREADS = 256;
-constexpr int BK = 64;
-
-__device__ __forceinline__ int sw(int r, int c) { return c ^ ((r >> 1) & 7); }
-
-template <int BM, int BN, int WM, int WN, int EPI>
-__global__ __launch_bounds__(THREADS) void gemm_kernel(const bf16_t* __restrict__ x, int ldx,
-                                                       const bf16_t* __restrict__ w, int M, int N, int K,
-                                                       bf16_t* y, int ldy) {
-    constexpr int TM = BM / WM, TN = BN / WN;
-    constexpr int FM = TM / 16, FN = TN / 16;
-    constexpr int XCH = BM * 8, WCH = BN * 8;  // 16-byte chunks per tile
-    constexpr int XPT = (XCH + THREADS - 1) / THREADS, WPT = (WCH + THREADS - 1) / THREADS;
-    static_assert(WM * WN == 4, "4 waves");
-
-    __shared__ __align__(16) bf16_t xs[BM * BK];
-    __shared__ __align__(16) bf16_t ws[BN * BK];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, n = lane & 15;
-    const int wm = wave / WN, wn = wave % WN;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-
-    uint4 xr[XPT], wr[WPT];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int j = 0; j < XPT; ++j) {
-            const int e = tid + j * THREADS;
-            const int r = e >> 3, c = e & 7;
-            xr[j] = make_uint4(0, 0, 0, 0);
-            if (e < XCH && m0 + r < M)
-                xr[j] = *reinterpret_cast<const uint4*>(x + (int64_t)(m0 + r) * ldx + k0 + 8 * c);
-        }
-#pragma unroll
-        for (int j = 0; j < WPT; ++j) {
-            const int e = tid + j * THREADS;
-            const int r = e >> 3, c = e & 7;
-            wr[j] = make_uint4(0, 0, 0, 0);
-            if (e < WCH && n0 + r < N)
-                wr[j] = load_nt((w + (int64_t)(n0 + r) * K + k0 + 8 * c));
-        }
-    };
-    auto sstore = [&]() {
-#pragma unroll
-        for (int j = 0; j < XPT; ++j) {
-            const int e = tid + j * THREADS;
-            if (e < XCH) {
-                const int r = e >> 3, c = e & 7;
-                *reinterpret_cast<uint4*>(xs + r * BK + sw(r, c) * 8) = xr[j];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < WPT; ++j) {
-            const int e = tid + j * THREADS;
-            if (e < WCH) {
-                const int r = e >> 3, c = e & 7;
-                *reinterpret_cast<uint4*>(ws + r * BK + sw(r, c) * 8) = wr[j];
-            }
-        }
-    };
-
-    f32x4_t acc[FN][FM];
-#pragma unroll
-    for (int i = 0; i < FN; ++i)
-#pragma unroll
-        for (int j = 0; j < FM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-    gload(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        __syncthreads();
-        sstore();
-        __syncthreads();
-        if (k0 + BK < K) gload(k0 + BK);
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            u32x4_t av[FN], bv[FM];
-#pragma unroll
-            for (int i = 0; i < FN; ++i) {
-                const int r = wn * TN + 16 * i + n;
-                av[i] = *reinterpret_cast<const u32x4_t*>(ws + r * BK + sw(r, 4 * kk + g) * 8);
-            }
-#pragma unroll
-            for (int j = 0; j < FM; ++j) {
-                const int r = wm * TM + 16 * j + n;
-                bv[j] = *reinterpret_cast<const u32x4_t*>(xs + r * BK + sw(r, 4 * kk + g) * 8);
-            }
-#pragma unroll
-            for (int i = 0; i < FN; ++i)
-#pragma unroll
-                for (int j = 0; j < FM; ++j) acc[i][j] = mfma(av[i], bv[j], acc[i][j]);
-        }
-    }
-
-    // acc[i][j][e] = C[token m0 + TM*wm + 16j + n][column n0 + TN*wn + 16i + 4g + e].
-#pragma unroll
-    for (int j = 0; j < FM; ++j) {
-        const int m = m0 + wm * TM + 16 * j + n;
-        if (m >= M) continue;
-#pragma unroll
-        for (int i = 0; i < FN; ++i) {
-            const int col = n0 + wn * TN + 16 * i + 4 * g;
-            if (col < N) store4<EPI>(y, ldy, m, col, acc[i][j]);
-        }
-    }
-}
-
-template <int BM, int BN, int WM, int WN>
-int launch(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y, int ldy,
-           hipStream_t stream) {
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-    switch (epi) {
-        case Q3_EPI_STORE:
-            Q3_LAUNCH((gemm_kernel<BM, BN, WM, WN, Q3_EPI_STORE>), grid, dim3(THREADS), 0, stream, x, ldx, w, M, N,
-                      K, y, ldy);
-            break;
-        case Q3_EPI_RESID:
-            Q3_LAUNCH((gemm_kernel<BM, BN, WM, WN, Q3_EPI_RESID>), grid, dim3(THREADS), 0, stream, x, ldx, w, M, N,
-                      K, y, ldy);
-            break;
-        case Q3_EPI_SWIGLU:
-            Q3_LAUNCH((gemm_kernel<BM, BN, WM, WN, Q3_EPI_SWIGLU>), grid, dim3(THREADS), 0, stream, x, ldx, w, M, N,
-                      K, y, ldy);
-            break;
-        default:
-            return (int)hipErrorInvalidValue;
-    }
-    Q3_CHECK_LAUNCH();
-}
-
 // Whole tiles 0..full-1, then the rest split `splits` ways (EPI_PARTIAL:
 // full == 0, partials [splits, M, N]; other epilogues: compact partials
 // finished by wide_tail_reduce_kernel, launched here after the GEMM).
@@ -537,35 +378,6 @@ int launch_wide(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, 
 
 }  // namespace
 
-// The wide tiling once it has at least this many 256 x 256 tiles (with fewer,
-// too many CUs would idle; measured on MI355X the 128 x 128 tiling is then
-// faster) and at least one full token tile (a 64-row LM head would waste
-// three quarters of each tile's MFMA work).
-constexpr int WIDE_MIN_TILES = 160;
-
-extern "C" int q3_gemm_tiles_wide(int M, int N) {
-    if (M < 256 || N < 1) return 0;
-    const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-    return tiles >= WIDE_MIN_TILES && tiles <= (1 << 30);
-}
-
-extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y,
-                       int ldy, hipStream_t stream) {
-    if (M < 1 || N < 4 || N % 4 || K < BK || K % BK || ldx % 8 || ldx < K || ldy % 4 || !x || !w || !y ||
-        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) ||
-        (reinterpret_cast<uintptr_t>(y) & 7))
-        return (int)hipErrorInvalidValue;
-    // A token tile's rows lie within 32-bit byte offsets of its first row.
-    if ((int64_t)256 * ldx * 2 > INT32_MAX || (int64_t)256 * K * 2 > INT32_MAX) return (int)hipErrorInvalidValue;
-    if (q3_gemm_tiles_wide(M, N))
-        return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, ((M + 255) / 256) * ((N + 255) / 256), 1, nullptr,
-                           stream);
-    if (M <= 16) return launch<16, 64, 1, 4>(x, ldx, w, M, N, K, epi, y, ldy, stream);
-    if (M <= 32) return launch<32, 64, 2, 2>(x, ldx, w, M, N, K, epi, y, ldy, stream);
-    if (M <= 64) return launch<64, 64, 2, 2>(x, ldx, w, M, N, K, epi, y, ldy, stream);
-    return launch<128, 128, 2, 2>(x, ldx, w, M, N, K, epi, y, ldy, stream);
-}
-
 // Compute units of the current device (cached per device; 0 if unknown).
 static int cu_count() {
     constexpr int MAX_DEV = 64;
@@ -580,17 +392,46 @@ static int cu_count() {
     return cached[dev] > 0 ? cached[dev] : 0;
 }
 
+// The wide tiling once it has at least this many 256 x 256 tiles (with fewer,
+// too many CUs would idle: o unsplit at 1000 tokens, 40 tiles, takes 34 us on
+// the mid tiling) and at least one full token tile (a 64-row LM head would
+// waste three quarters of each tile's MFMA work).
+constexpr int WIDE_MIN_TILES = 160;
+
+static int mid_cus() {
+    const int cus = cu_count();
+    return cus > 0 ? cus : 256;
+}
+
+extern "C" int q3_gemm_tiles_wide(int M, int N) {
+    if (M < 256 || N < 1) return 0;
+    const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
+    return tiles >= WIDE_MIN_TILES && tiles <= (1 << 30);
+}
+
+extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y,
+                       int ldy, hipStream_t stream) {
+    if (M < 1 || N < 4 || N % 4 || K < WIDE_BK || K % WIDE_BK || ldx % 8 || ldx < K || ldy % 4 || !x || !w || !y ||
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) ||
+        (reinterpret_cast<uintptr_t>(y) & 7))
+        return (int)hipErrorInvalidValue;
+    // A token tile's rows lie within 32-bit byte offsets of its first row.
+    if ((int64_t)256 * ldx * 2 > INT32_MAX || (int64_t)256 * K * 2 > INT32_MAX) return (int)hipErrorInvalidValue;
+    if (q3_gemm_tiles_wide(M, N))
+        return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, ((M + 255) / 256) * ((N + 255) / 256), 1, nullptr,
+                           stream);
+    return launch_mid(mid_plan(M, N, K, mid_cus(), 1), x, ldx, w, M, N, K, epi, y, ldy, nullptr, stream);
+}
+
 // Split tail of the wide tiling.  One 256 x 256-tile workgroup fits a CU
 // (128 KB of LDS), so the tiles run in rounds of `cus`; when the last round
 // is at most half full, its tiles are split along K over about `cus`
 // workgroups (at most TAIL_MAX_SPLITS splits of >= WIDE_SPLIT_STEPS K
 // steps), which shortens that round by the split count, and
 // wide_tail_reduce_kernel finishes them.  Below WIDE_MIN_TILES the same
-// applies to all the tiles when they fill at most half the CUs (from 256
-// tokens; measured against the 128 x 128 tiling: qkv at 512 / 768 / 1024
-// tokens 50.7 / 59.1 / 61.8 -> 37.5 / 42.4 / 52.8 us, gate/up at 256 tokens
-// 61.8 -> 48.5).  The partials take tail * splits <= cus tiles of 256 x 256
-// FP32.
+// applies to all the tiles when they fill at most half the CUs, from
+// MID_MAX_TOKENS on (qkv at 1000 tokens 51.0 us, 53.6 on the mid tiling).  The
+// partials take tail * splits <= cus tiles of 256 x 256 FP32.
 struct WidePlan {
     int full, tail, splits;
 };
@@ -610,8 +451,20 @@ static WidePlan wide_tail_plan(int M, int N, int K) {
     return {tiles - rem, rem, s};
 }
 
+// Token counts up to here take the mid tiling wherever whole 256 x 256 tiles do
+// not fill the CUs, in place of split ones (measured, us, split tail -> mid:
+// qkv at 300 / 384 / 512 tokens 33.4 / 35.0 / 38.7 -> 23.6 / 26.4 / 30.3, o
+// 29.9 / 31.1 / 32.8 -> 22 / 22.5 / 25.5, gate/up 60.0 / 61.3 / 93.2 -> 57.0 /
+// 61.5 / 84.3; at 1000 tokens gate/up takes 107, 159 on the mid tiling).
+constexpr int MID_MAX_TOKENS = 512;
+
 extern "C" int q3_gemm_ws_floats(int M, int N, int K) {
     if (M < 1 || N < 4 || K < WIDE_BK || K % WIDE_BK) return 0;
+    if (M < 256) {
+        const MidPlan p = mid_plan(M, N, K, mid_cus(), MID_MAX_SPLITS);
+        const int64_t floats = p.splits > 1 ? (int64_t)p.splits * M * N : 0;
+        return floats <= INT32_MAX ? (int)floats : 0;
+    }
     const WidePlan p = wide_tail_plan(M, N, K);
     return p.tail * p.splits * 256 * 256;
 }
@@ -619,14 +472,19 @@ extern "C" int q3_gemm_ws_floats(int M, int N, int K) {
 extern "C" int q3_gemm_ws(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y,
                           int ldy, float* ws, hipStream_t stream) {
     const int need = q3_gemm_ws_floats(M, N, K);
-    if (need == 0 || epi == EPI_PARTIAL) return q3_gemm(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    if (need == 0 || epi == EPI_PARTIAL || (M < 256 && !ws)) return q3_gemm(x, ldx, w, M, N, K, epi, y, ldy, stream);
     if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15)) return (int)hipErrorInvalidValue;
-    // The operand checks of q3_gemm, which would take the same wide path.
+    // The operand checks of q3_gemm.
     if (N % 4 || ldx % 8 || ldx < K || ldy % 4 || !x || !w || !y ||
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) ||
         (reinterpret_cast<uintptr_t>(y) & 7))
         return (int)hipErrorInvalidValue;
     if ((int64_t)256 * ldx * 2 > INT32_MAX || (int64_t)256 * K * 2 > INT32_MAX) return (int)hipErrorInvalidValue;
+    if (M <= MID_MAX_TOKENS && !q3_gemm_tiles_wide(M, N)) {
+        const int64_t fit = need / ((int64_t)M * N);  // splits whose partials the workspace holds
+        const int most = (int)(fit < 1 ? 1 : fit < MID_MAX_SPLITS ? fit : MID_MAX_SPLITS);
+        return launch_mid(mid_plan(M, N, K, mid_cus(), most), x, ldx, w, M, N, K, epi, y, ldy, ws, stream);
+    }
     const WidePlan p = wide_tail_plan(M, N, K);
     return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, p.full, p.splits, ws, stream);
 }

@@ -1,0 +1,360 @@
+// Dense BF16 projection for token counts too small for the 256 x 256 tiling:
+// decode batches above 64 rows and prompts up to a few hundred tokens.
+//
+// y[m, n] = epi(sum_k x[m, k] * W[n, k]).  At 9-512 tokens a projection moves
+// about as many bytes of activations through each CU as of weights, and both
+// far outweigh the arithmetic, so the kernel is built around two streams that
+// never wait for each other:
+//   * weights go from HBM (row-major, 128 bytes of a row per step of 64 K)
+//     straight into MFMA A operands, MID_RING - 1 steps ahead in registers;
+//     each weight row is read by one wave, which holds 16 * NB of them.  The
+//     two load instructions of a step each take half of 16 lines; plain loads,
+//     so that the second finds its halves in L1, which non-temporal ones fetch
+//     again (measured at 16 tokens, gate/up: 26.3 -> 21.0 us, qkv 9.9 -> 6.9;
+//     whole lines per instruction, 20.1, would sum K in another order than the
+//     256 x 256 tiling does);
+//   * the 16 * MB token rows of a step are filled into LDS by loader waves
+//     with direct global-to-LDS loads, MID_STAGES - 1 steps ahead, and feed
+//     every compute wave as B operands.  Waves of their own, because vector
+//     memory counters retire in order: a compute wave that loaded both would
+//     wait for its newest token rows with every weight it needs.  One wave
+//     streams at most ~27 GB/s whatever its depth, four ~100 GB/s, hence the
+//     loader counts (gate/up at 250 tokens: two loaders 57 us, four 45).
+// A workgroup is NW compute waves (16 NB NW weight rows) and the loader waves,
+// one barrier per step; with split > 1 the workgroups of a tile take
+// contiguous K ranges and mid_reduce_kernel sums their FP32 partials in split
+// order and applies the epilogue.
+//
+// What bounds it: the weights' HBM stream (5.0 TB/s at 16 tokens on gate/up,
+// against 6.8 for a plain copy-in) and, from ~64 tokens on, the LDS reads of
+// the token rows, 16 MB * 128 bytes per step and compute wave.  Measured
+// against the register-staged 128 x 128 tiling that it replaced (us, cold
+// weights, splits included): 45 tokens qkv 36.6 -> 11.6, o 56.7 -> 10.7,
+// gate/up 40.3 -> 23.6, down 131 -> 15.0; 100 tokens 47.5 -> 14.1, 73.7 ->
+// 13.7, 50.0 -> 30.7, 169 -> 20.1; o unsplit at 1000 tokens 76 -> 35.
+#pragma once
+
+#include "q3_common.hpp"
+#include "q3_dma.hpp"
+#include "q3.h"
+
+namespace q3gemm {
+
+using namespace q3dma;
+
+constexpr int EPI_PARTIAL = -1;  // FP32 split partials, no rounding
+
+__device__ __forceinline__ f32x4_t mfma(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                   c, 0, 0, 0);
+}
+
+// Four consecutive output columns col..col+3 of token row m (col % 4 == 0).
+template <int EPI>
+__device__ __forceinline__ void store4(bf16_t* y, int ldy, int m, int col, const f32x4_t& v) {
+    if constexpr (EPI == Q3_EPI_SWIGLU) {
+        const uint32_t a = pack_bf16x2(v[0], v[1]), b = pack_bf16x2(v[2], v[3]);  // gate, up rounded
+        *reinterpret_cast<uint32_t*>(y + (int64_t)m * ldy + (col >> 1)) =
+            pack_bf16x2(silu_bf16(bflo(a)) * bfhi(a), silu_bf16(bflo(b)) * bfhi(b));
+    } else {
+        uint2* p = reinterpret_cast<uint2*>(y + (int64_t)m * ldy + col);
+        if constexpr (EPI == Q3_EPI_RESID) {
+            const uint2 r = *p;
+            const uint32_t a = pack_bf16x2(v[0], v[1]), b = pack_bf16x2(v[2], v[3]);
+            *p = make_uint2(pack_bf16x2(bflo(r.x) + bflo(a), bfhi(r.x) + bfhi(a)),
+                            pack_bf16x2(bflo(r.y) + bflo(b), bfhi(r.y) + bfhi(b)));
+        } else {
+            *p = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        }
+    }
+}
+
+// Position of 16-byte chunk c of 128-byte row r: c ^ ((r >> 1) & 7).  Measured
+// on gfx950: a ds_read_b128 whose 64 lanes read rows r0..r0+15 at one logical
+// chunk (four k groups) runs at the linear-read rate; no swizzle is 2.5x slower.
+__device__ __forceinline__ int wide_swz(int r) { return (r >> 1) & 7; }
+
+constexpr int MID_BK = 64;     // K elements of a step: 128 bytes of a row
+constexpr int MID_STAGES = 6;  // LDS stages of token rows
+constexpr int MID_RING = 4;    // register sets of weights
+constexpr int MID_LEAD = 4;    // LDS reads ahead of their MFMAs
+
+struct MidArgs {
+    const bf16_t* x;
+    int ldx;
+    const bf16_t* w;
+    int M, N, K;
+    int epi;        // Q3_EPI_* or EPI_PARTIAL
+    bf16_t* y;
+    int ldy;
+    float* part;    // [splits, M, N] (EPI_PARTIAL)
+    int tm, tn;     // token and weight tiles
+    int splits;
+};
+
+// Loader waves: one per SIMD where the token rows of a step are most of the
+// bytes (an odd count of 16-row blocks does not deal out over four).
+template <int MB>
+constexpr int MID_LOADERS = MB > 4 ? (MB % 2 ? 2 : 4) : MB > 1 ? 2 : 1;
+
+template <int MB, int NB, int NW>
+__global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(MidArgs a) {
+    constexpr int LW = MID_LOADERS<MB>, PER = 2 * MB / LW, XT = 16 * MB * 128;  // XT: bytes of a stage
+    constexpr int AHEAD = MID_STAGES - 1;
+    static_assert(2 * MB % LW == 0 && PER * AHEAD <= 63, "direct loads in flight exceed the vmcnt range");
+    __shared__ __align__(1024) char lds[MID_STAGES * XT];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    // Workgroup b runs on XCD b % 8: give each XCD a contiguous range, token
+    // tiles fastest, so the workgroups that share weight rows share an L2.
+    const int total = gridDim.x, xcd = blockIdx.x & 7, q = total >> 3, rem = total & 7;
+    const int v = xcd * q + min(xcd, rem) + (int)(blockIdx.x >> 3);
+    const int mt = v % a.tm, nt = (v / a.tm) % a.tn, split = v / (a.tm * a.tn);
+    const int m0 = mt * 16 * MB, n0 = nt * 16 * NB * NW;
+    const int steps = a.K / MID_BK;
+    const int nk = steps / a.splits + (split < steps % a.splits ? 1 : 0);
+    const int kb = (split * (steps / a.splits) + min(split, steps % a.splits)) * MID_BK;
+
+    if (wave >= NW) {
+        // Direct load i of loader wave lw fills rows 8d..8d+7 of the stage, d =
+        // lw + LW i: lane l the chunk position l % 8 of row 8d + l / 8.  Rows
+        // past M re-read the last row: in bounds, results not stored.
+        const int lw = wave - NW;
+        const bf16_t* xb = a.x + (int64_t)m0 * a.ldx + kb;
+        uint32_t voff[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int r = 8 * (lw + LW * i) + (lane >> 3);
+            voff[i] = (uint32_t)((min(m0 + r, a.M - 1) - m0) * a.ldx + 8 * ((lane & 7) ^ wide_swz(r))) * 2u;
+        }
+        const uint32_t lbase = lds_address(lds) + 1024 * lw;
+        auto issue = [&](int c) {
+            const bf16_t* xc = xb + min(c, nk - 1) * MID_BK;
+            const uint32_t sbase = lbase + (uint32_t)(c % MID_STAGES) * XT;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) load_to_lds(xc, voff[i], sbase + 1024 * LW * i);
+        };
+#pragma unroll
+        for (int c = 0; c < AHEAD; ++c) issue(c);
+        wait_vmcnt<PER * (AHEAD - 1)>();
+        __syncthreads();
+        for (int c = 0; c + 1 < nk; ++c) {
+            // Stage (c + AHEAD) % MID_STAGES was last read in step c - 1, which
+            // every wave finished before the barrier that ended it.
+            issue(c + AHEAD);
+            wait_vmcnt<PER * (AHEAD - 1)>();  // step c + 1 landed
+            __syncthreads();
+        }
+        wait_vmcnt<0>();  // no direct-to-LDS load may land after the workgroup ends
+        return;
+    }
+
+    const int g = lane >> 4, n = lane & 15;
+    const int row0 = n0 + wave * 16 * NB;
+    const bf16_t* wr[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) wr[i] = a.w + (int64_t)min(row0 + 16 * i + n, a.N - 1) * a.K + kb + 8 * g;
+    u32x4_t wv[MID_RING][NB][2];
+    auto load = [&](int c, u32x4_t (&d)[NB][2]) {
+        const int k = min(c, nk - 1) * MID_BK;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+                d[i][kk] = *reinterpret_cast<const u32x4_t*>(wr[i] + k + 32 * kk);
+    };
+    f32x4_t acc[NB][MB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // Token row 16j + n (same swizzle as row n), logical chunk 4kk + g.
+    int boff[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) boff[kk] = (n * 8 + ((4 * kk + g) ^ wide_swz(n))) * 16;
+
+#pragma unroll
+    for (int c = 0; c < MID_RING - 1; ++c) load(c, wv[c]);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    // LDS reads run MID_LEAD operands ahead of their MFMAs; the compiler's own
+    // order waits for each right before its use (gate/up at 100 tokens 32.5 ->
+    // 30.7 us).
+    constexpr int LEAD = MB < MID_LEAD ? MB : MID_LEAD;
+    auto step = [&](int c, int u) {
+        const char* xp = lds + (c % MID_STAGES) * XT;
+        u32x4_t b[2][MB];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int j = 0; j < MB; ++j) b[kk][j] = *reinterpret_cast<const u32x4_t*>(xp + boff[kk] + j * 16 * 128);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int j = 0; j < MB; ++j)
+#pragma unroll
+                for (int i = 0; i < NB; ++i) acc[i][j] = mfma(wv[u][i][kk], b[kk][j], acc[i][j]);
+        __builtin_amdgcn_sched_group_barrier(0x100, LEAD, 0);  // LDS reads
+#pragma unroll
+        for (int q = 0; q < 2 * MB - LEAD; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, NB, 0);  // MFMAs
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, LEAD * NB, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Groups of MID_RING steps, each step first loading the one MID_RING - 1
+    // ahead; the last group (1..MID_RING steps) has its steps in flight but one.
+    int c0 = 0;
+    for (; nk - c0 > MID_RING; c0 += MID_RING) {
+#pragma unroll
+        for (int u = 0; u < MID_RING; ++u) {
+            load(c0 + u + MID_RING - 1, wv[(u + MID_RING - 1) % MID_RING]);
+            // Keep the prefetch here: the scheduler would otherwise sink each
+            // load down to its use and the MFMAs would wait for fresh loads.
+            __builtin_amdgcn_sched_barrier(0);
+            step(c0 + u, u);
+            __syncthreads();
+        }
+    }
+    load(c0 + MID_RING - 1, wv[MID_RING - 1]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < MID_RING; ++u) {
+        if (c0 + u < nk) step(c0 + u, u);
+        if (c0 + u + 1 < nk) __syncthreads();
+    }
+
+    // acc[i][j][e] = C[token m0 + 16j + n][column row0 + 16i + 4g + e].
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+        const int m = m0 + 16 * j + n;
+        if (m >= a.M) continue;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int col = row0 + 16 * i + 4 * g;
+            if (col >= a.N) continue;
+            if (a.epi == EPI_PARTIAL)
+                *reinterpret_cast<f32x4_t*>(a.part + ((int64_t)split * a.M + m) * a.N + col) = acc[i][j];
+            else if (a.epi == Q3_EPI_SWIGLU)
+                store4<Q3_EPI_SWIGLU>(a.y, a.ldy, m, col, acc[i][j]);
+            else if (a.epi == Q3_EPI_RESID)
+                store4<Q3_EPI_RESID>(a.y, a.ldy, m, col, acc[i][j]);
+            else
+                store4<Q3_EPI_STORE>(a.y, a.ldy, m, col, acc[i][j]);
+        }
+    }
+}
+
+// Sum of the split partials in split order, then the epilogue; thread: four
+// columns of one token row.  Every split's load is issued before the sum.
+constexpr int MID_MAX_SPLITS = 8;
+
+template <int EPI>
+__global__ __launch_bounds__(256) void mid_reduce_kernel(const float* __restrict__ part, int splits, int M, int N,
+                                                         bf16_t* y, int ldy) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int quads = N / 4;
+    if (e >= (int64_t)M * quads) return;
+    const int m = (int)(e / quads), c = 4 * (int)(e % quads);
+    const float* src = part + (int64_t)m * N + c;
+    const int64_t stride = (int64_t)M * N;
+    f32x4_t p[MID_MAX_SPLITS];
+#pragma unroll
+    for (int s = 0; s < MID_MAX_SPLITS; ++s)
+        p[s] = *reinterpret_cast<const f32x4_t*>(src + min(s, splits - 1) * stride);
+    f32x4_t v = p[0];
+#pragma unroll
+    for (int s = 1; s < MID_MAX_SPLITS; ++s)
+        if (s < splits) v += p[s];
+    store4<EPI>(y, ldy, m, c, v);
+}
+
+// Launch shape: MB token blocks x NB NW weight blocks of 16 per workgroup, and
+// the K splits.
+struct MidPlan {
+    int mb, nb, nw, splits;
+};
+
+// The tile shapes that are built, as NB, NW.
+constexpr int MID_SHAPES[][2] = {{1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 3}, {2, 5}, {2, 8}};
+constexpr int MID_MAX_MB = 8;
+constexpr int MID_MIN_SPLIT_STEPS = 4;  // K steps of a split, at least
+
+// Picks the plan of least estimated time.  A CU's bytes set it, not its
+// arithmetic, so a step costs about 20 ns per 16-row block that the workgroup
+// loads (weights or tokens) plus 100 ns of barrier and latency, once per round
+// of workgroups over the CUs; splitting adds its partials' traffic (write and
+// read at 5 TB/s) and the reduce launch (4.5 us).  Against a sweep of all
+// shapes at 12-1000 tokens on the four projections the pick is the fastest or
+// within 8% of it (o at 512 tokens 26.0 against 23.8 us at worst).
+inline MidPlan mid_plan(int M, int N, int K, int cus, int max_splits) {
+    const int steps = K / MID_BK, mblocks = (M + 15) / 16, nblocks = (N + 15) / 16;
+    MidPlan best{1, 1, 2, 1};
+    double best_us = 1e30;
+    for (const auto& sh : MID_SHAPES) {
+        const int wb = sh[0] * sh[1];
+        for (int mb = mblocks < MID_MAX_MB ? mblocks : MID_MAX_MB; mb >= 1; --mb) {
+            const int64_t tiles = (int64_t)((mblocks + mb - 1) / mb) * ((nblocks + wb - 1) / wb);
+            const double rounds = (double)((tiles + cus - 1) / cus);
+            // Splits only within one round of workgroups.
+            for (int s = 1; s == 1 || (s <= max_splits && tiles * s <= cus && steps >= s * MID_MIN_SPLIT_STEPS); ++s) {
+                double us = 0.02 * (5 + wb + mb) * ((steps + s - 1) / s) * rounds;
+                if (s > 1) us += 4.5 + (double)s * M * N * 8.0 / 5e6;
+                if (us < best_us) {
+                    best_us = us;
+                    best = {mb, sh[0], sh[1], s};
+                }
+            }
+        }
+    }
+    return best;
+}
+
+template <int MB>
+int launch_mid_mb(const MidPlan& p, const MidArgs& a, hipStream_t stream) {
+    const dim3 grid((unsigned)(a.tm * a.tn * a.splits));
+    switch (p.nb * 10 + p.nw) {
+#define Q3_MID(nb, nw)                                                                                           \
+    case nb * 10 + nw:                                                                                           \
+        Q3_LAUNCH((gemm_mid_kernel<MB, nb, nw>), grid, dim3((nw + MID_LOADERS<MB>) * 64), 0, stream, a);         \
+        return (int)hipGetLastError();
+        Q3_MID(1, 2) Q3_MID(1, 3) Q3_MID(1, 4) Q3_MID(1, 5) Q3_MID(2, 3) Q3_MID(2, 5) Q3_MID(2, 8)
+#undef Q3_MID
+    }
+    return (int)hipErrorInvalidValue;
+}
+
+// y = epi(x . W^T) under plan p; part holds [p.splits, M, N] floats when
+// p.splits > 1.
+inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi,
+                      bf16_t* y, int ldy, float* part, hipStream_t stream) {
+    if (epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU) return (int)hipErrorInvalidValue;
+    if (p.splits > 1 && (!part || p.splits > MID_MAX_SPLITS)) return (int)hipErrorInvalidValue;
+    const int tm = (M + 16 * p.mb - 1) / (16 * p.mb), tn = (N + 16 * p.nb * p.nw - 1) / (16 * p.nb * p.nw);
+    if ((int64_t)tm * tn * p.splits > (1 << 30)) return (int)hipErrorInvalidValue;
+    const MidArgs a{x, ldx, w, M, N, K, p.splits > 1 ? EPI_PARTIAL : epi, y, ldy, part, tm, tn, p.splits};
+    int rc = (int)hipErrorInvalidValue;
+    switch (p.mb) {
+        case 1: rc = launch_mid_mb<1>(p, a, stream); break;
+        case 2: rc = launch_mid_mb<2>(p, a, stream); break;
+        case 3: rc = launch_mid_mb<3>(p, a, stream); break;
+        case 4: rc = launch_mid_mb<4>(p, a, stream); break;
+        case 5: rc = launch_mid_mb<5>(p, a, stream); break;
+        case 6: rc = launch_mid_mb<6>(p, a, stream); break;
+        case 7: rc = launch_mid_mb<7>(p, a, stream); break;
+        case 8: rc = launch_mid_mb<8>(p, a, stream); break;
+    }
+    if (rc || p.splits == 1) return rc;
+    const dim3 grid((unsigned)(((int64_t)M * (N / 4) + 255) / 256));
+    if (epi == Q3_EPI_SWIGLU)
+        Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_SWIGLU>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);
+    else if (epi == Q3_EPI_RESID)
+        Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_RESID>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);
+    else
+        Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_STORE>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);
+    Q3_CHECK_LAUNCH();
+}
+
+}  // namespace q3gemm

@@ -37,7 +37,7 @@ Decode step (one hipGraph, self-feeding like reference ``:805-839``), B <= 8:
 For B > GEMV_BATCH_MAX the projections stream 16-row tiled weight copies into
 MFMA (B <= 64), their split-K partials summed by the consuming kernel (the
 attention prologue, the residual add + RMSNorm); above 64 rows, or for shapes
-that do not tile, the LDS-tiled MFMA GEMM with separate norm kernels.
+that do not tile, the short-prompt MFMA GEMM with separate norm kernels.
 """
 
 from __future__ import annotations
@@ -73,7 +73,7 @@ MEMORY_MARGIN_BYTES = 2 << 30
 #: Largest decode batch on the dot2 GEMVs (fused norm prologue and argmax
 #: epilogue).  Above it, up to SKINNY_BATCH_MAX, projections stream 16-row
 #: tiled weight copies into MFMA (``q3_skinny_tiled``), which at 5+ rows beats
-#: the GEMV's VALU-bound dot products; above that the LDS-tiled GEMM.
+#: the GEMV's VALU-bound dot products; above that the short-prompt GEMM.
 GEMV_BATCH_MAX = 4
 SKINNY_BATCH_MAX = 64
 
@@ -334,6 +334,11 @@ class Engine:
             for N, K in self._projections():
                 ws = max(ws, call("q3_skinny_splits", B, N, K) * B * N)
         self.skinny_ws = self._empty(max(ws, 1), dtype=torch.float32)
+        # Split partials of the other MFMA decode projections (more than 64 rows).
+        ws = 0
+        if not self.small and not self.skinny:
+            ws = max(call("q3_gemm_ws_floats", B, N, K) for N, K in self._projections())
+        self.proj_ws = self._empty(max(ws, 1), dtype=torch.float32)
         if self.small:
             self.lm_parts = call("q3_gemv_partials", B, V, _lib.EPI_ARGMAX)
         elif self.skinny:
@@ -546,8 +551,9 @@ class Engine:
 
     def _proj(self, x: int, ldx: int, w: torch.Tensor, N: int, K: int, epi: int, y: int, ldy: int) -> None:
         """Decode projection for batches outside the GEMV and fused MFMA paths (more
-        than 64 rows, or shapes that do not tile): the LDS-tiled MFMA GEMM."""
-        call("q3_gemm", x, ldx, _ptr(w), self.batch, N, K, epi, y, ldy, self._s)
+        than 64 rows, or shapes that do not tile): the short-prompt MFMA GEMM,
+        long K split over workgroups (down at 100 rows: 30.5 us unsplit, 18.8 split)."""
+        call("q3_gemm_ws", x, ldx, _ptr(w), self.batch, N, K, epi, y, ldy, _ptr(self.proj_ws), self._s)
 
     def _capture(self) -> None:
         """Warm every kernel eagerly, then record one decode step as a hipGraph.

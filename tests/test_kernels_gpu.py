@@ -355,6 +355,47 @@ def test_gemm(M, N, K):
     assert_nearly_exact(act, oc.swiglu(yc[:, 0::2], yc[:, 1::2]), frac=5e-3)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 32, 64), (15, 36, 192), (16, 2560, 4096), (17, 2560, 9728), (33, 260, 320),
+                                   (45, 2560, 9728), (81, 84, 576), (127, 6144, 2560), (128, 2560, 9728),
+                                   (129, 1028, 832), (255, 2560, 4096), (257, 3800, 448), (511, 516, 64)])
+def test_gemm_short_prompt_tiles(M, N, K):
+    """The loader-wave tiling of q3_gemm / q3_gemm_ws below the 256 x 256 one: token and weight tiles that end
+    inside a 16-row block, one K step up to more than a register ring, splits with uneven K ranges (the 2560-wide
+    long-K shapes).  Sampled rows against float64; nothing written past N or M; both epilogues of the split path
+    bit-exact against its own stored projection."""
+    assert call("q3_gemm_tiles_wide", M, N) == 0
+    x, w = rnd((M, K), 1.0, M + 61), rnd((N, K), 0.02, N + K + 61)
+    xd, wd = dv(x), dv(w)
+    floats = call("q3_gemm_ws_floats", M, N, K)
+    assert floats > 0 or (N, K) != (2560, 9728)  # the down projection's shape splits K
+    ws = dv(torch.full((floats + 64,), 9.0, dtype=torch.float32))
+    g = torch.Generator().manual_seed(M)
+    rows = torch.cat([torch.tensor([0, M - 1]), torch.randint(0, M, (30,), generator=g)])
+
+    def ld(cols):  # rows of the output padded to a multiple of four, at least four past the columns
+        return (cols + 7) // 4 * 4
+
+    def run(name, epi, cols, fill, *tail):
+        out = dv(fill.clone())
+        call(name, P(xd), K, P(wd), M, N, K, epi, P(out), ld(cols), *tail, S())
+        torch.cuda.synchronize()
+        out = out.cpu()
+        assert torch.equal(out[:, cols:], fill[:, cols:]) and torch.equal(out[M:], fill[M:])
+        return out[:M, :cols].contiguous()
+
+    for name, tail in (("q3_gemm", ()), ("q3_gemm_ws", (P(ws),))):
+        y = run(name, _lib.EPI_STORE, N, torch.full((M + 2, ld(N)), 5.0, dtype=torch.bfloat16), *tail)
+        check_projection(y[rows], x[rows], w)
+        res = torch.full((M + 2, ld(N)), 5.0, dtype=torch.bfloat16)
+        res[:M, :N] = rnd((M, N), 1.0, 63)
+        joined = run(name, _lib.EPI_RESID, N, res, *tail)
+        assert torch.equal(joined, (res[:M, :N].float() + y.float()).bfloat16())
+        act = run(name, _lib.EPI_SWIGLU, N // 2, torch.full((M + 2, ld(N // 2)), 5.0, dtype=torch.bfloat16),
+                  *tail)
+        assert_nearly_exact(act, oc.swiglu(y[:, 0::2], y[:, 1::2]), frac=5e-3)
+    assert torch.all(ws.cpu()[floats:] == 9.0)
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(4096, 6144, 2560, _lib.EPI_STORE), (4096, 2560, 4096, _lib.EPI_RESID),
                                        (2600, 19456, 2560, _lib.EPI_SWIGLU), (4096, 2560, 9728, _lib.EPI_RESID),
                                        (3000, 3800, 320, _lib.EPI_STORE), (40961, 4096, 64, _lib.EPI_STORE)])
