@@ -182,6 +182,27 @@ def test_gemv_plain_store(M, N, K):
     check_projection(y, x, w)
 
 
+@pytest.mark.parametrize("M", [3, 4])
+@pytest.mark.parametrize("N,K", [(1, 2560), (30, 2560), (333, 2560), (6151, 2560), (2555, 9728), (2557, 4096)])
+def test_gemv_three_and_four_rows(M, N, K):
+    """Three and four rows: the MFMA kernel of K = 2560 (row counts that are no multiple of its four rows per wave,
+    waves past the last row, six- and eight-wave workgroups) and the ten-wave dot2 workgroups of the long K, plain and
+    with the residual join, nothing written past a row's N columns."""
+    x, w, res = rnd((M, K), 1.0, M), rnd((N, K), 0.02, N + K), rnd((M, N + 8), 1.0, 7)
+    xd, wd = dv(x), dv(w)
+    y = dv(torch.full((M, N + 8), 5.0, dtype=torch.bfloat16))
+    joined = dv(res.clone())
+    for epi, out in ((_lib.EPI_STORE, y), (_lib.EPI_RESID, joined)):
+        call("q3_gemv", _lib.X_PLAIN, P(xd), K, None, None, 0.0, None, P(wd), M, N, K, epi, P(out), N + 8,
+             None, None, None, None, None, 0, S())
+    torch.cuda.synchronize()
+    yc, jc = y.cpu(), joined.cpu()
+    # A third of the outputs round like float64 at least at N = 1 (three or four values).
+    check_projection(yc[:, :N], x, w, frac=0.03 if N > 100 else 0.34)
+    assert torch.all(yc[:, N:] == 5.0) and torch.equal(jc[:, N:], res[:, N:])
+    assert torch.equal(jc[:, :N], (res[:, :N].float() + yc[:, :N].float()).bfloat16())
+
+
 def gemv(x_mode, x, ldx, w, M, N, K, epi, y, ldy, ids=None, norm_w=None, resid_out=None, pv=None, pi=None,
          pos=None, feed=None, rec=None):
     call("q3_gemv", x_mode, P(x), ldx, P(ids), P(norm_w), 1e-6, P(resid_out), P(w), M, N, K, epi, P(y), ldy,
