@@ -288,15 +288,24 @@ constexpr int MID_MIN_SPLIT_STEPS = 4;  // K steps of a split, at least
 // of workgroups over the CUs; splitting adds its partials' traffic (write and
 // read at 5 TB/s) and the reduce launch (4.5 us).  Against a sweep of all
 // shapes at 12-1000 tokens on the four projections the pick is the fastest or
-// within 8% of it (o at 512 tokens 26.0 against 23.8 us at worst).
-inline MidPlan mid_plan(int M, int N, int K, int cus, int max_splits) {
+// within 8% of it (o at 512 tokens 26.0 against 23.8 us at worst).  With
+// fixed_splits, the best tile for that many splits.
+inline MidPlan mid_plan(int M, int N, int K, int cus, int max_splits, int fixed_splits = 0) {
     const int steps = K / MID_BK, mblocks = (M + 15) / 16, nblocks = (N + 15) / 16;
-    MidPlan best{1, 1, 2, 1};
+    MidPlan best{1, 1, 2, fixed_splits ? fixed_splits : 1};
     double best_us = 1e30;
     for (const auto& sh : MID_SHAPES) {
         const int wb = sh[0] * sh[1];
         for (int mb = mblocks < MID_MAX_MB ? mblocks : MID_MAX_MB; mb >= 1; --mb) {
             const int64_t tiles = (int64_t)((mblocks + mb - 1) / mb) * ((nblocks + wb - 1) / wb);
+            if (fixed_splits) {
+                const double us = 0.02 * (5 + wb + mb) * (double)((tiles * fixed_splits + cus - 1) / cus);
+                if (us < best_us) {
+                    best_us = us;
+                    best = {mb, sh[0], sh[1], fixed_splits};
+                }
+                continue;
+            }
             const double rounds = (double)((tiles + cus - 1) / cus);
             // Splits only within one round of workgroups.
             for (int s = 1; s == 1 || (s <= max_splits && tiles * s <= cus && steps >= s * MID_MIN_SPLIT_STEPS); ++s) {
@@ -327,11 +336,14 @@ int launch_mid_mb(const MidPlan& p, const MidArgs& a, hipStream_t stream) {
 }
 
 // y = epi(x . W^T) under plan p; part holds [p.splits, M, N] floats when
-// p.splits > 1.
+// p.splits > 1 or epi is EPI_PARTIAL (which leaves the sum to the caller).
 inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi,
                       bf16_t* y, int ldy, float* part, hipStream_t stream) {
-    if (epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU) return (int)hipErrorInvalidValue;
-    if (p.splits > 1 && (!part || p.splits > MID_MAX_SPLITS)) return (int)hipErrorInvalidValue;
+    const bool partial = epi == EPI_PARTIAL;
+    if (!partial && epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU)
+        return (int)hipErrorInvalidValue;
+    if ((p.splits > 1 || partial) && !part) return (int)hipErrorInvalidValue;
+    if (p.splits > MID_MAX_SPLITS && !partial) return (int)hipErrorInvalidValue;
     const int tm = (M + 16 * p.mb - 1) / (16 * p.mb), tn = (N + 16 * p.nb * p.nw - 1) / (16 * p.nb * p.nw);
     if ((int64_t)tm * tn * p.splits > (1 << 30)) return (int)hipErrorInvalidValue;
     const MidArgs a{x, ldx, w, M, N, K, p.splits > 1 ? EPI_PARTIAL : epi, y, ldy, part, tm, tn, p.splits};
@@ -346,7 +358,7 @@ inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* 
         case 7: rc = launch_mid_mb<7>(p, a, stream); break;
         case 8: rc = launch_mid_mb<8>(p, a, stream); break;
     }
-    if (rc || p.splits == 1) return rc;
+    if (rc || partial || p.splits == 1) return rc;
     const dim3 grid((unsigned)(((int64_t)M * (N / 4) + 255) / 256));
     if (epi == Q3_EPI_SWIGLU)
         Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_SWIGLU>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);

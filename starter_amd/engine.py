@@ -646,6 +646,14 @@ class Engine:
             self._prefill_part = self._empty(floats, dtype=torch.float32)
         return self._prefill_part
 
+    def _residual_splits(self, M: int, K: int) -> int:
+        """K splits of a residual projection over M prompt tokens whose partials
+        the residual add + RMSNorm sums; 0 where it is not split."""
+        s = call("q3_gemm_splits", M, self.HIDDEN, K)
+        if not s and M < 256:  # the short-prompt tiling's own count
+            s = call("q3_gemm_ws_floats", M, self.HIDDEN, K) // (M * self.HIDDEN)
+        return s
+
     def _forward_prefill(self, ids: torch.Tensor, seq_len: int) -> torch.Tensor:
         """Consume the prompt ``ids [B, P]``; return the last position's logits [B, 1, V].
 
@@ -684,8 +692,7 @@ class Engine:
                 # residual projections along K; their partials are summed (in split
                 # order), joined to the residual and normalised by one row kernel,
                 # which replaces the RMSNorm that follows each of them.
-                s_o = call("q3_gemm_splits", M, H, self.q_size)
-                s_d = call("q3_gemm_splits", M, H, I)
+                s_o, s_d = self._residual_splits(M, self.q_size), self._residual_splits(M, I)
                 # Longer prompts whose last round of tiles is at most half full split
                 # those tiles along K (q3_gemm_ws); the same buffer holds either.
                 floats = max(s_o, s_d) * M * H

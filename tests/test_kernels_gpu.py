@@ -541,6 +541,28 @@ def test_gemm_partials(M, N, K):
         assert_nearly_exact(y, oc.rms_norm(want, gain, 1e-6), max_ulp=2)
 
 
+@pytest.mark.parametrize("M,N,K,splits", [(1, 36, 192, 3), (17, 260, 704, 2), (45, 2560, 9728, 8), (100, 2560, 4096, 16),
+                                          (129, 1028, 832, 5), (255, 2560, 9728, 1)])
+def test_gemm_partials_short_prompt(M, N, K, splits):
+    """q3_gemm_partials below 256 tokens, on the short-prompt tiling: ragged token and weight tiles, uneven K ranges
+    and one step per split; the partials summed in split order against float64 on sampled rows, nothing written past
+    splits * M * N floats."""
+    x, w = rnd((M, K), 1.0, M + 71), rnd((N, K), 0.02, N + K + 71)
+    xd, wd = dv(x), dv(w)
+    ws = dv(torch.full((splits * M * N + 4 * N,), 9.0))
+    call("q3_gemm_partials", P(xd), K, P(wd), M, N, K, P(ws), splits, S())
+    torch.cuda.synchronize()
+    part = ws.cpu()
+    assert torch.all(part[splits * M * N:] == 9.0)
+    part = part[:splits * M * N].view(splits, M, N)
+    acc = part[0].clone()
+    for s_ in range(1, splits):
+        acc += part[s_]
+    g = torch.Generator().manual_seed(M)
+    rows = torch.cat([torch.tensor([0, M - 1]), torch.randint(0, M, (30,), generator=g)])
+    check_projection(acc[rows].bfloat16(), x[rows], w)
+
+
 def wide_origin(t, tm, tn):
     """Tile t's (token, weight-row) origin in the 256 x 256 tiling's raster order."""
     per_group = 4 * tn
