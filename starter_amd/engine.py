@@ -665,7 +665,10 @@ class Engine:
         if B != self.batch or seq_len > self.capacity or ids.shape[1] != seq_len:
             raise ValueError(f"prefill of {tuple(ids.shape)} does not fit the cache "
                              f"(batch {self.batch}, capacity {self.capacity})")
-        if int(ids.min()) < 0 or int(ids.max()) >= self.VOCAB:
+        # One reduction and one copy back for both bounds (ids on the device
+        # would take two of each, with the GPU idle meanwhile).
+        lo, hi = torch.stack(torch.aminmax(ids)).tolist()
+        if lo < 0 or hi >= self.VOCAB:
             raise ValueError(f"token ids must lie in [0, {self.VOCAB})")
         if ids.is_cuda:
             # Made on the caller's stream, read on ours: keep the block alive until
