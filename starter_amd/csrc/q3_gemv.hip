@@ -153,53 +153,65 @@ __device__ void stage_x(const GemvArgs& a, bf16_t* xs) {
 // for them does not wait for the weights (vector memory counters retire in
 // order), and the norm / copy runs while the weights are still in flight.
 // Arithmetic and order are those of stage_x.
+// Eight-wave workgroups stage X_NORM rows in two four-wave groups, the second
+// half of the rows by the second: norm_groups(W) groups of norm_rows<M, W>
+// rows, each row's arithmetic that of four waves.
+constexpr int norm_groups(int W) { return W == 2 * GEMV_WAVES ? 2 : 1; }
+template <int M, int XMODE, int W>
+constexpr int stage_rows = XMODE == Q3_X_NORM ? (M + norm_groups(W) - 1) / norm_groups(W) : M;
+template <int XMODE, int W>
+constexpr int stage_threads = XMODE == Q3_X_NORM ? GEMV_THREADS : W * Q3_WAVE;
+
 template <int XMODE, int KU, int W>
 constexpr int x_chunks() {
-    return (64 * KU + W * Q3_WAVE - 1) / (W * Q3_WAVE);
+    return (64 * KU + stage_threads<XMODE, W> - 1) / stage_threads<XMODE, W>;
 }
 
 template <int M, int XMODE, int KU, int W>
-__device__ __forceinline__ void stage_x_issue(const GemvArgs& a, u32x4_t (&xv)[x_chunks<XMODE, KU, W>()][M],
+__device__ __forceinline__ void stage_x_issue(const GemvArgs& a,
+                                              u32x4_t (&xv)[x_chunks<XMODE, KU, W>()][stage_rows<M, XMODE, W>],
                                               u32x4_t (&gv)[x_chunks<XMODE, KU, W>()]) {
-    constexpr int XC = x_chunks<XMODE, KU, W>();
-    const int tid = threadIdx.x;
+    constexpr int XC = x_chunks<XMODE, KU, W>(), MG = stage_rows<M, XMODE, W>, NT = stage_threads<XMODE, W>;
+    const int tid = threadIdx.x % NT, m0 = threadIdx.x / NT * MG;
 #pragma unroll
     for (int j = 0; j < XC; ++j) {
-        const int c = min(tid + j * W * Q3_WAVE, 64 * KU - 1);  // past the row: a duplicate, never used
+        const int c = min(tid + j * NT, 64 * KU - 1);  // past the row: a duplicate, never used
         if constexpr (XMODE == Q3_X_NORM) gv[j] = *reinterpret_cast<const u32x4_t*>(a.norm_w + c * 8);
 #pragma unroll
-        for (int m = 0; m < M; ++m) xv[j][m] = *reinterpret_cast<const u32x4_t*>(a.x + (int64_t)m * a.ldx + c * 8);
+        for (int m = 0; m < MG; ++m)
+            xv[j][m] = *reinterpret_cast<const u32x4_t*>(a.x + (int64_t)min(m0 + m, M - 1) * a.ldx + c * 8);
     }
 }
 
 template <int M, int XMODE, int KU, int W>
-__device__ __forceinline__ void stage_x_finish(const GemvArgs& a, const u32x4_t (&xv)[x_chunks<XMODE, KU, W>()][M],
+__device__ __forceinline__ void stage_x_finish(const GemvArgs& a,
+                                               const u32x4_t (&xv)[x_chunks<XMODE, KU, W>()][stage_rows<M, XMODE, W>],
                                                const u32x4_t (&gv)[x_chunks<XMODE, KU, W>()], bf16_t* xs) {
-    constexpr int XC = x_chunks<XMODE, KU, W>();
+    constexpr int XC = x_chunks<XMODE, KU, W>(), MG = stage_rows<M, XMODE, W>, NT = stage_threads<XMODE, W>;
     constexpr int K = 512 * KU;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x % NT, grp = threadIdx.x / NT, m0 = grp * MG;
     if constexpr (XMODE == Q3_X_PLAIN) {
 #pragma unroll
         for (int j = 0; j < XC; ++j) {
-            const int c = tid + j * W * Q3_WAVE;
+            const int c = tid + j * NT;
             if (c < 64 * KU)
 #pragma unroll
                 for (int m = 0; m < M; ++m) *reinterpret_cast<u32x4_t*>(xs + m * K + c * 8) = xv[j][m];
         }
         __syncthreads();
     } else {
-        static_assert(XMODE == Q3_X_NORM && W == GEMV_WAVES, "norm staging is written for four waves");
+        static_assert(XMODE == Q3_X_NORM && W == norm_groups(W) * GEMV_WAVES, "norm staging is by groups of four waves");
         const int lane = tid & 63, wave = tid >> 6;
-        __shared__ float red[GEMV_WAVES][M];
-        float ss[M];
+        __shared__ float red[norm_groups(W)][GEMV_WAVES][MG];
+        float ss[MG];
 #pragma unroll
-        for (int m = 0; m < M; ++m) ss[m] = 0.f;
+        for (int m = 0; m < MG; ++m) ss[m] = 0.f;
 #pragma unroll
         for (int j = 0; j < XC; ++j) {
-            const int c = tid + j * W * Q3_WAVE;
+            const int c = tid + j * NT;
             if (c < 64 * KU) {
 #pragma unroll
-                for (int m = 0; m < M; ++m) {
+                for (int m = 0; m < MG; ++m) {
                     const u32x4_t v = xv[j][m];
                     float s = ss[m];
                     s += bflo(v.x) * bflo(v.x); s += bfhi(v.x) * bfhi(v.x);
@@ -211,31 +223,32 @@ __device__ __forceinline__ void stage_x_finish(const GemvArgs& a, const u32x4_t 
             }
         }
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
+        for (int m = 0; m < MG; ++m) {
             float s = wave_sum(ss[m]);
-            if (lane == 0) red[wave][m] = s;
+            if (lane == 0) red[grp][wave][m] = s;
         }
         __syncthreads();
-        float inv[M];
+        float inv[MG];
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            float s = (red[0][m] + red[1][m]) + (red[2][m] + red[3][m]);
+        for (int m = 0; m < MG; ++m) {
+            float s = (red[grp][0][m] + red[grp][1][m]) + (red[grp][2][m] + red[grp][3][m]);
             inv[m] = inv_rms(s, K, a.eps);
         }
 #pragma unroll
         for (int j = 0; j < XC; ++j) {
-            const int c = tid + j * W * Q3_WAVE;
+            const int c = tid + j * NT;
             if (c < 64 * KU) {
                 const u32x4_t g = gv[j];
 #pragma unroll
-                for (int m = 0; m < M; ++m) {
+                for (int m = 0; m < MG; ++m) {
+                    if (m0 + m >= M) continue;
                     u32x4_t v = xv[j][m];
                     const float im = inv[m];
                     v.x = pack2(norm_elem(bflo(v.x), im, bflo(g.x)), norm_elem(bfhi(v.x), im, bfhi(g.x)));
                     v.y = pack2(norm_elem(bflo(v.y), im, bflo(g.y)), norm_elem(bfhi(v.y), im, bfhi(g.y)));
                     v.z = pack2(norm_elem(bflo(v.z), im, bflo(g.z)), norm_elem(bfhi(v.z), im, bfhi(g.z)));
                     v.w = pack2(norm_elem(bflo(v.w), im, bflo(g.w)), norm_elem(bfhi(v.w), im, bfhi(g.w)));
-                    *reinterpret_cast<u32x4_t*>(xs + m * K + c * 8) = v;
+                    *reinterpret_cast<u32x4_t*>(xs + (m0 + m) * K + c * 8) = v;
                 }
             }
         }
@@ -350,7 +363,7 @@ __global__ __launch_bounds__(W * Q3_WAVE) void gemv_dot2_kernel(GemvArgs a) {
         // Input rows first unless they come from the embedding (ids first).
         constexpr bool SPLIT = XLDS && XMODE != Q3_X_EMBED_NORM;
         constexpr int XC = x_chunks<XMODE, KU, W>();
-        u32x4_t xv[XC][M], gv[XC];
+        u32x4_t xv[XC][stage_rows<M, XMODE, W>], gv[XC];
         if constexpr (SPLIT) stage_x_issue<M, XMODE, KU, W>(a, xv, gv);
         __builtin_amdgcn_sched_barrier(0);  // keep the input loads ahead of the weight loads
         // No load under a condition (a wave past the last row re-reads the
@@ -404,207 +417,6 @@ __global__ __launch_bounds__(W * Q3_WAVE) void gemv_dot2_kernel(GemvArgs a) {
     }
 }
 
-// ------------------------------------------------- three and four rows, MFMA
-//
-// At three or four batch rows the dot products themselves cost: 4 M dot2 per
-// 16 weight bytes and M LDS reads, on top of the same stream (gate/up 13.9 us
-// at one row, 19.8 at three, 23 at four).  v_mfma_f32_4x4x4_16b_bf16 takes the
-// four rows at the price of one: sixteen independent blocks, each 4 weight
-// rows x 4 batch rows x 4 K.  Lane (b, i), b = lane / 4, i = lane % 4, loads 16
-// bytes of weight row i at chunk b of a 128-element K piece (each load
-// instruction: 256 contiguous bytes of four rows) and reads the same chunk of
-// batch row i from LDS; D[row r][batch row i] of block b is its acc[r], and
-// the sixteen blocks' sums meet once at the end.  K = 2560, where a wave's 20
-// loads (80 registers) are all in flight before the prologue.
-constexpr int MK = 2560;            // K of this kernel
-constexpr int MLOADS = MK / 128;    // 16-byte weight loads per lane
-// Loads in flight per lane: all of them, but twelve in ten-wave workgroups, whose
-// five waves per SIMD (two workgroups a CU) then fit the registers.
-constexpr int mfma_flight(int W) { return W == 10 ? 12 : MLOADS; }
-constexpr int MXLD = MK + 32;       // LDS row pitch: the four batch rows of a read on different banks
-
-// Input rows of this thread's four-wave group: m0 .. m0 + MG - 1 (clamped to
-// the last), chunks tid and tid + 256 of each (the second clamped to the
-// row's last).  Arithmetic and order are stage_x's.
-template <int MG>
-struct NormRows {
-    u32x4_t xv[2][MG], gv[2];
-};
-
-template <int M, int MG, int XMODE>
-__device__ __forceinline__ void norm_rows_issue(const GemvArgs& a, int m0, int tid, NormRows<MG>& r) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int c = min(tid + j * GEMV_THREADS, MK / 8 - 1);
-        if constexpr (XMODE != Q3_X_PLAIN) r.gv[j] = *reinterpret_cast<const u32x4_t*>(a.norm_w + c * 8);
-#pragma unroll
-        for (int m = 0; m < MG; ++m) {
-            const int row = min(m0 + m, M - 1);
-            const bf16_t* src = a.x + (XMODE == Q3_X_EMBED_NORM ? a.ids[row] * (int64_t)MK : (int64_t)row * a.ldx);
-            r.xv[j][m] = *reinterpret_cast<const u32x4_t*>(src + c * 8);
-        }
-    }
-}
-
-template <int M, int MG, int XMODE, int GROUPS>
-__device__ __forceinline__ void norm_rows_finish(const GemvArgs& a, int m0, int tid, bool stager, const NormRows<MG>& r,
-                                                 bf16_t* xs) {
-    const int lane = tid & 63, wave = tid >> 6, grp = m0 / MG;
-    __shared__ float red[GROUPS][GEMV_WAVES][MG];
-    if constexpr (XMODE != Q3_X_PLAIN) {
-        if (stager) {
-#pragma unroll
-            for (int m = 0; m < MG; ++m) {
-                float s = 0.f;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    if (tid + j * GEMV_THREADS >= MK / 8) continue;
-                    const u32x4_t v = r.xv[j][m];
-                    s += bflo(v.x) * bflo(v.x); s += bfhi(v.x) * bfhi(v.x);
-                    s += bflo(v.y) * bflo(v.y); s += bfhi(v.y) * bfhi(v.y);
-                    s += bflo(v.z) * bflo(v.z); s += bfhi(v.z) * bfhi(v.z);
-                    s += bflo(v.w) * bflo(v.w); s += bfhi(v.w) * bfhi(v.w);
-                }
-                s = wave_sum(s);
-                if (lane == 0) red[grp][wave][m] = s;
-            }
-        }
-        __syncthreads();
-    }
-    if (stager) {
-#pragma unroll
-        for (int m = 0; m < MG; ++m) {
-            if (m0 + m >= M) continue;
-            float inv = 0.f;
-            if constexpr (XMODE != Q3_X_PLAIN)
-                inv = inv_rms((red[grp][0][m] + red[grp][1][m]) + (red[grp][2][m] + red[grp][3][m]), MK, a.eps);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int c = tid + j * GEMV_THREADS;
-                if (c >= MK / 8) continue;
-                u32x4_t v = r.xv[j][m];
-                if (XMODE == Q3_X_EMBED_NORM && blockIdx.x == 0)
-                    *reinterpret_cast<u32x4_t*>(a.resid_out + (int64_t)(m0 + m) * MK + c * 8) = v;
-                if constexpr (XMODE != Q3_X_PLAIN) {
-                    const u32x4_t g = r.gv[j];
-                    v.x = pack2(norm_elem(bflo(v.x), inv, bflo(g.x)), norm_elem(bfhi(v.x), inv, bfhi(g.x)));
-                    v.y = pack2(norm_elem(bflo(v.y), inv, bflo(g.y)), norm_elem(bfhi(v.y), inv, bfhi(g.y)));
-                    v.z = pack2(norm_elem(bflo(v.z), inv, bflo(g.z)), norm_elem(bfhi(v.z), inv, bfhi(g.z)));
-                    v.w = pack2(norm_elem(bflo(v.w), inv, bflo(g.w)), norm_elem(bfhi(v.w), inv, bfhi(g.w)));
-                }
-                *reinterpret_cast<u32x4_t*>(xs + (m0 + m) * MXLD + c * 8) = v;
-            }
-        }
-    }
-    __syncthreads();
-}
-
-// W waves of four weight rows.  The first four waves stage the input rows; of
-// eight waves, the second four stage the second half of them.
-template <int M, int XMODE, int EPI, int W>
-__global__ __launch_bounds__(W * Q3_WAVE, W == 10 ? 5 : 1) void gemv_mfma_kernel(GemvArgs a) {
-    static_assert(M == 3 || M == 4, "four batch rows per MFMA block");
-    constexpr bool ARGMAX = EPI == Q3_EPI_ARGMAX || EPI == Q3_EPI_STORE_ARGMAX;
-    static_assert(!ARGMAX || W == GEMV_WAVES, "the argmax epilogue is written for four waves");
-    constexpr int GROUPS = W >= 2 * GEMV_WAVES ? 2 : 1, MG = GROUPS == 2 ? 2 : M;
-    __shared__ __align__(16) bf16_t xs[M * MXLD];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = lane >> 2, i = lane & 3;
-    const int row0 = (blockIdx.x * W + wave) * 4;
-    const bool stager = wave < GROUPS * GEMV_WAVES;
-    const int tid = threadIdx.x & (GEMV_THREADS - 1), m0 = GROUPS == 2 ? (wave >> 2) * MG : 0;
-
-    NormRows<MG> rows;
-    norm_rows_issue<M, MG, XMODE>(a, m0, tid, rows);
-    __builtin_amdgcn_sched_barrier(0);  // keep the input loads ahead of the weight loads
-    const bf16_t* wp = a.w + (int64_t)min(row0 + i, a.N - 1) * MK + b * 8;
-    constexpr int NF = mfma_flight(W);
-    uint4 wv[NF];
-#pragma unroll
-    for (int u = 0; u < NF; ++u) wv[u] = load_nt(wp + u * 128);
-    __builtin_amdgcn_sched_barrier(0);  // and these weight loads issued before the prologue
-    norm_rows_finish<M, MG, XMODE, GROUPS>(a, m0, tid, stager, rows, xs);
-
-    typedef short i16x4_t __attribute__((ext_vector_type(4)));
-    const bf16_t* xp = xs + min(i, M - 1) * MXLD + b * 8;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < MLOADS; ++u) {
-        const uint4 xv = *reinterpret_cast<const uint4*>(xp + u * 128);
-        const uint4 w4 = wv[u % NF];
-        acc = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(i16x4_t, make_uint2(w4.x, w4.y)),
-                                                     __builtin_bit_cast(i16x4_t, make_uint2(xv.x, xv.y)), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(i16x4_t, make_uint2(w4.z, w4.w)),
-                                                     __builtin_bit_cast(i16x4_t, make_uint2(xv.z, xv.w)), acc, 0, 0, 0);
-        if (u + NF < MLOADS) {
-            wv[u % NF] = load_nt(wp + (u + NF) * 128);
-            if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    // Sum over the blocks: the lanes of equal i, within the 16-lane rows and
-    // across them.
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        float v = acc[r];
-        v += Q3_DPP(v, 0x124);  // row_ror:4
-        v += Q3_DPP(v, 0x128);  // row_ror:8
-        v += __shfl_xor(v, 16, Q3_WAVE);
-        v += __shfl_xor(v, 32, Q3_WAVE);
-        acc[r] = v;
-    }
-    const bool active = row0 < a.N;
-    if constexpr (EPI != Q3_EPI_ARGMAX) {
-        if (lane < M && active) {
-            const int m = lane;
-            if constexpr (EPI == Q3_EPI_SWIGLU) {
-                bf16_t* p = a.y + (int64_t)m * a.ldy + (row0 >> 1);
-                p[0] = (bf16_t)f2bf(silu_bf16(rbf(acc[0])) * rbf(acc[1]));
-                p[1] = (bf16_t)f2bf(silu_bf16(rbf(acc[2])) * rbf(acc[3]));
-            } else {
-                bf16_t* p = a.y + (int64_t)m * a.ldy + row0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (row0 + r >= a.N) continue;
-                    p[r] = EPI == Q3_EPI_RESID ? (bf16_t)f2bf(bf2f(p[r]) + rbf(acc[r])) : (bf16_t)f2bf(acc[r]);
-                }
-            }
-        }
-    }
-    if constexpr (ARGMAX) {
-        float all[4][M];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-                all[r][m] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc[r]), m));
-        argmax_epilogue<M, 4>(a, all, row0, active, lane, wave);
-    }
-}
-
-template <int M, int XMODE, int EPI, int W>
-int launch_mfma_w(const GemvArgs& a, hipStream_t stream) {
-    Q3_LAUNCH((gemv_mfma_kernel<M, XMODE, EPI, W>), dim3((a.N + 4 * W - 1) / (4 * W)), dim3(W * Q3_WAVE), 0, stream, a);
-    Q3_CHECK_LAUNCH();
-}
-
-// Waves per workgroup: four for the argmax epilogue; ten for SwiGLU (19456
-// rows: 487 workgroups, all resident, each staging the rows once: 19.2 / 20.7
-// us at three / four rows against 20.0 / 21.0 with eight waves); six where
-// they deal the rows out evenly over the CUs and eight do not (6144 rows: 256
-// workgroups, 7.7 / 8.1 us against 8.2 / 8.6); else eight.
-template <int M, int XMODE, int EPI>
-int launch_mfma(const GemvArgs& a, hipStream_t stream) {
-    if constexpr (EPI == Q3_EPI_ARGMAX || EPI == Q3_EPI_STORE_ARGMAX) {
-        return a.N % 4 == 0 ? launch_mfma_w<M, XMODE, EPI, GEMV_WAVES>(a, stream) : -1;
-    } else {
-        if constexpr (EPI == Q3_EPI_SWIGLU)
-            return a.N % 4 == 0 ? launch_mfma_w<M, XMODE, EPI, 10>(a, stream) : -1;
-        auto most = [&](int w) { return ((a.N + 4 * w - 1) / (4 * w) + 255) / 256 * w; };  // waves of the busiest CU
-        if (most(6) < most(8)) return launch_mfma_w<M, XMODE, EPI, 6>(a, stream);
-        return launch_mfma_w<M, XMODE, EPI, 8>(a, stream);
-    }
-}
-
 // Rows per wave.  Projections: one row per wave, so the N rows spread over N
 // waves and every CU streams.  SwiGLU takes two (gate, up) pairs: gate_up's
 // 19456 rows then make 1216 workgroups, all resident at once (two rows per
@@ -629,7 +441,8 @@ constexpr bool combo_used(int xmode, int epi) {
 // spreads the rows more evenly over the 256 CUs (N = 2560: 512 workgroups,
 // two per CU, against 640 = 2.5 per CU with four).  From three batch rows on
 // ten waves do the same with one staging of the rows per CU instead of two
-// (K = 9728: they are 58 KB at three rows, 78 at four).
+// (K = 9728: they are 58 KB at three rows, 78 at four; 12.0 / 15.0 -> 10.9 /
+// 12.1 us).
 int waves_for(int xmode, int epi, int M, int N) {
     constexpr int CUS = 256;
     if (xmode != Q3_X_PLAIN || epi == Q3_EPI_ARGMAX || epi == Q3_EPI_STORE_ARGMAX) return GEMV_WAVES;
@@ -659,6 +472,13 @@ int launch_one(const GemvArgs& a, hipStream_t stream) {
         }
         if (w >= 5) return launch_w<M, KU, XMODE, XLDS, EPI, 5>(a, stream);
     }
+    // Stored normed projections of two rows on: eight waves share one staging
+    // (us, four -> eight waves, rows 2 / 3 / 4: 6144 rows 8.7 / 10.5 / 12.5 ->
+    // 7.7 / 9.0 / 10.1; 151936 rows 120 / 167 / 230 -> 110 / 135 / 155).  SwiGLU,
+    // four rows a wave, is slower so (17.4 / 18.9 / 21.5 -> 19.1 / 24.0 / 26.1).
+    if constexpr (XMODE == Q3_X_NORM && KU > 0 && M >= 2 && EPI == Q3_EPI_STORE) {
+        return launch_w<M, KU, XMODE, XLDS, EPI, 2 * GEMV_WAVES>(a, stream);
+    }
     return launch_w<M, KU, XMODE, XLDS, EPI, GEMV_WAVES>(a, stream);
 }
 
@@ -676,9 +496,6 @@ int launch_ku(const GemvArgs& a, hipStream_t stream) {
 
 template <int M, int XMODE, int EPI>
 int launch_rows(const GemvArgs& a, hipStream_t stream) {
-    if constexpr (combo_used(XMODE, EPI) && (M == 3 || M == 4)) {
-        if (a.K == MK) return launch_mfma<M, XMODE, EPI>(a, stream);
-    }
     if constexpr (!combo_used(XMODE, EPI)) {
         return -1;
     } else if constexpr (XMODE != Q3_X_PLAIN) {

@@ -182,25 +182,32 @@ def test_gemv_plain_store(M, N, K):
     check_projection(y, x, w)
 
 
-@pytest.mark.parametrize("M", [3, 4])
-@pytest.mark.parametrize("N,K", [(1, 2560), (30, 2560), (333, 2560), (6151, 2560), (2555, 9728), (2557, 4096)])
-def test_gemv_three_and_four_rows(M, N, K):
-    """Three and four rows: the MFMA kernel of K = 2560 (row counts that are no multiple of its four rows per wave,
-    waves past the last row, six- and eight-wave workgroups) and the ten-wave dot2 workgroups of the long K, plain and
-    with the residual join, nothing written past a row's N columns."""
+@pytest.mark.parametrize("M", [2, 3, 4, 5])
+@pytest.mark.parametrize("N,K", [(1, 2560), (333, 2560), (6151, 2560), (2555, 9728), (2557, 4096)])
+def test_gemv_large_workgroups(M, N, K):
+    """Ten-wave workgroups (plain input, three and four rows, the 2560-wide long-K shapes) and eight-wave ones (X_NORM,
+    two groups of four waves staging half the rows each), with waves past the last row: the plain projection against
+    float64, the residual join and the normed projection bit for bit against it, nothing written past N columns."""
     x, w, res = rnd((M, K), 1.0, M), rnd((N, K), 0.02, N + K), rnd((M, N + 8), 1.0, 7)
-    xd, wd = dv(x), dv(w)
-    y = dv(torch.full((M, N + 8), 5.0, dtype=torch.bfloat16))
-    joined = dv(res.clone())
-    for epi, out in ((_lib.EPI_STORE, y), (_lib.EPI_RESID, joined)):
-        call("q3_gemv", _lib.X_PLAIN, P(xd), K, None, None, 0.0, None, P(wd), M, N, K, epi, P(out), N + 8,
+    xd, wd, g = dv(x), dv(w), dv((1 + rnd((K,), 0.2, 8).float()).to(torch.bfloat16))
+    n = dv(torch.empty(M, K, dtype=torch.bfloat16))
+    outs = [dv(torch.full((M, N + 8), 5.0, dtype=torch.bfloat16)) for _ in range(3)] + [dv(res.clone())]
+    normed_too = K <= 4096  # the norm prologue's limit
+    if normed_too:
+        call("q3_rmsnorm", P(xd), K, P(g), P(n), K, M, K, 1e-6, S())
+    for mode, src, epi, out in ((_lib.X_PLAIN, xd, _lib.EPI_STORE, outs[0]), (_lib.X_PLAIN, n, _lib.EPI_STORE, outs[1]),
+                                (_lib.X_NORM, xd, _lib.EPI_STORE, outs[2]), (_lib.X_PLAIN, xd, _lib.EPI_RESID, outs[3])):
+        if not normed_too and (src is n or mode == _lib.X_NORM):
+            continue
+        call("q3_gemv", mode, P(src), K, None, P(g), 1e-6, None, P(wd), M, N, K, epi, P(out), N + 8,
              None, None, None, None, None, 0, S())
     torch.cuda.synchronize()
-    yc, jc = y.cpu(), joined.cpu()
-    # A third of the outputs round like float64 at least at N = 1 (three or four values).
-    check_projection(yc[:, :N], x, w, frac=0.03 if N > 100 else 0.34)
-    assert torch.all(yc[:, N:] == 5.0) and torch.equal(jc[:, N:], res[:, N:])
-    assert torch.equal(jc[:, :N], (res[:, :N].float() + yc[:, :N].float()).bfloat16())
+    plain, plain_n, normed, joined = (o.cpu() for o in outs)
+    check_projection(plain[:, :N], x, w, frac=0.03 if N > 100 else 0.5)  # N = 1: two to five values
+    assert torch.all(plain[:, N:] == 5.0) and torch.equal(joined[:, N:], res[:, N:])
+    assert torch.equal(joined[:, :N], (res[:, :N].float() + plain[:, :N].float()).bfloat16())
+    if normed_too:
+        assert torch.equal(normed, plain_n)
 
 
 def gemv(x_mode, x, ldx, w, M, N, K, epi, y, ldy, ids=None, norm_w=None, resid_out=None, pv=None, pi=None,
