@@ -91,9 +91,8 @@ int q3_gemm_tiles_wide(int M, int N);
  * ws [splits, M, N] (splits * M * N floats), summed in split order by
  * q3_add_rmsnorm_partials.  q3_gemm_splits(M, N, K) is the split count where
  * that applies (else 0); q3_gemm_partials takes any M and any splits in
- * 1..min(16, K / 64) (below 256 tokens on the short-prompt tiling, whose own
- * split count is q3_gemm_ws_floats(M, N, K) / (M * N)).  Same operand rules as
- * q3_gemm; ws 16-byte aligned. */
+ * 1..min(16, K / 64) (below 256 tokens on the short-prompt tiling).  Same
+ * operand rules as q3_gemm; ws 16-byte aligned. */
 int q3_gemm_splits(int M, int N, int K);
 int q3_gemm_partials(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
                      float *ws, int splits, hipStream_t stream);
@@ -105,8 +104,8 @@ int q3_gemm_partials(const uint16_t *x, int ldx, const uint16_t *w, int M, int N
  * the other tiles are q3_gemm's, bit for bit.  Below 256 tokens, projections
  * of long K may split K over all tiles the same way.  ws holds
  * q3_gemm_ws_floats(M, N, K) floats (0: nothing is split, and q3_gemm_ws is
- * q3_gemm), 16-byte aligned; up to 512 tokens it may be more than is used.
- * Same operand rules as q3_gemm. */
+ * q3_gemm), 16-byte aligned; below 256 tokens ws may be NULL (nothing is
+ * split).  Same operand rules as q3_gemm. */
 int q3_gemm_ws_floats(int M, int N, int K);
 int q3_gemm_ws(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
                int epi, uint16_t *y, int ldy, float *ws, hipStream_t stream);

@@ -429,9 +429,9 @@ extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, 
 // workgroups (at most TAIL_MAX_SPLITS splits of >= WIDE_SPLIT_STEPS K
 // steps), which shortens that round by the split count, and
 // wide_tail_reduce_kernel finishes them.  Below WIDE_MIN_TILES the same
-// applies to all the tiles when they fill at most half the CUs, from
-// MID_MAX_TOKENS on (qkv at 1000 tokens 51.0 us, 53.6 on the mid tiling).  The
-// partials take tail * splits <= cus tiles of 256 x 256 FP32.
+// applies to all the tiles when they fill at most half the CUs, from 256
+// tokens (qkv at 512 / 1000 tokens 38.7 / 51.0 us; whole on the mid tiling 30.3
+// / 53.6).  The partials take tail * splits <= cus tiles of 256 x 256 FP32.
 struct WidePlan {
     int full, tail, splits;
 };
@@ -450,13 +450,6 @@ static WidePlan wide_tail_plan(int M, int N, int K) {
     if (s < 2) return {tiles, 0, 1};
     return {tiles - rem, rem, s};
 }
-
-// Token counts up to here take the mid tiling wherever whole 256 x 256 tiles do
-// not fill the CUs, in place of split ones (measured, us, split tail -> mid:
-// qkv at 300 / 384 / 512 tokens 33.4 / 35.0 / 38.7 -> 23.6 / 26.4 / 30.3, o
-// 29.9 / 31.1 / 32.8 -> 22 / 22.5 / 25.5, gate/up 60.0 / 61.3 / 93.2 -> 57.0 /
-// 61.5 / 84.3; at 1000 tokens gate/up takes 107, 159 on the mid tiling).
-constexpr int MID_MAX_TOKENS = 512;
 
 extern "C" int q3_gemm_ws_floats(int M, int N, int K) {
     if (M < 1 || N < 4 || K < WIDE_BK || K % WIDE_BK) return 0;
@@ -480,11 +473,8 @@ extern "C" int q3_gemm_ws(const bf16_t* x, int ldx, const bf16_t* w, int M, int 
         (reinterpret_cast<uintptr_t>(y) & 7))
         return (int)hipErrorInvalidValue;
     if ((int64_t)256 * ldx * 2 > INT32_MAX || (int64_t)256 * K * 2 > INT32_MAX) return (int)hipErrorInvalidValue;
-    if (M <= MID_MAX_TOKENS && !q3_gemm_tiles_wide(M, N)) {
-        const int64_t fit = need / ((int64_t)M * N);  // splits whose partials the workspace holds
-        const int most = (int)(fit < 1 ? 1 : fit < MID_MAX_SPLITS ? fit : MID_MAX_SPLITS);
-        return launch_mid(mid_plan(M, N, K, mid_cus(), most), x, ldx, w, M, N, K, epi, y, ldy, ws, stream);
-    }
+    if (M < 256)  // need > 0: the plan splits K
+        return launch_mid(mid_plan(M, N, K, mid_cus(), MID_MAX_SPLITS), x, ldx, w, M, N, K, epi, y, ldy, ws, stream);
     const WidePlan p = wide_tail_plan(M, N, K);
     return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, p.full, p.splits, ws, stream);
 }

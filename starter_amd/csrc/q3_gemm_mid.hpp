@@ -6,13 +6,17 @@
 // far outweigh the arithmetic, so the kernel is built around two streams that
 // never wait for each other:
 //   * weights go from HBM (row-major, 128 bytes of a row per step of 64 K)
-//     straight into MFMA A operands, MID_RING - 1 steps ahead in registers;
-//     each weight row is read by one wave, which holds 16 * NB of them.  The
-//     two load instructions of a step each take half of 16 lines; plain loads,
-//     so that the second finds its halves in L1, which non-temporal ones fetch
-//     again (measured at 16 tokens, gate/up: 26.3 -> 21.0 us, qkv 9.9 -> 6.9;
-//     whole lines per instruction, 20.1, would sum K in another order than the
-//     256 x 256 tiling does);
+//     straight into MFMA A operands, two or three steps ahead in registers;
+//     each weight row is read by one wave, which holds 16 * NB of them.  An
+//     operand is 64 bytes of 16 rows.  With one token tile each weight is read
+//     once: a load instruction then takes whole 128-byte lines of eight rows,
+//     non-temporal (a plain streaming kernel reads 7.0 TB/s so, 6.1 with plain
+//     loads), and two DPP moves per register make operands of two loads.  With
+//     several token tiles the weights are shared through L2 and L1: plain loads
+//     in operand order, the second instruction of a line finding it in L1;
+//     non-temporal ones fetch the line again (gate/up at 16 tokens, us:
+//     non-temporal half lines 26.3, plain half lines 20.6, whole lines 18.2; at
+//     100 tokens 35.3 / 30.7 / 27.1);
 //   * the 16 * MB token rows of a step are filled into LDS by loader waves
 //     with direct global-to-LDS loads, MID_STAGES - 1 steps ahead, and feed
 //     every compute wave as B operands.  Waves of their own, because vector
@@ -25,13 +29,14 @@
 // contiguous K ranges and mid_reduce_kernel sums their FP32 partials in split
 // order and applies the epilogue.
 //
-// What bounds it: the weights' HBM stream (5.0 TB/s at 16 tokens on gate/up,
-// against 6.8 for a plain copy-in) and, from ~64 tokens on, the LDS reads of
-// the token rows, 16 MB * 128 bytes per step and compute wave.  Measured
+// What bounds it: the weights' HBM stream (5.5 TB/s at 16 tokens on gate/up,
+// launch included) and, from ~64 tokens on, the token rows beside it: without
+// them gate/up takes 21 us at 100 tokens, without the weights 10, without MFMAs
+// or LDS reads as long as with them.  Measured
 // against the register-staged 128 x 128 tiling that it replaced (us, cold
-// weights, splits included): 45 tokens qkv 36.6 -> 11.6, o 56.7 -> 10.7,
-// gate/up 40.3 -> 23.6, down 131 -> 15.0; 100 tokens 47.5 -> 14.1, 73.7 ->
-// 13.7, 50.0 -> 30.7, 169 -> 20.1; o unsplit at 1000 tokens 76 -> 35.
+// weights, splits included): 45 tokens qkv 36.6 -> 10.9, o 56.7 -> 10.4,
+// gate/up 40.3 -> 20.5, down 131 -> 14; 100 tokens 47.5 -> 14.1, 73.7 ->
+// 13.7, 50.0 -> 27.1, 169 -> 18; o unsplit at 1000 tokens 76 -> 35.
 #pragma once
 
 #include "q3_common.hpp"
@@ -76,7 +81,6 @@ __device__ __forceinline__ int wide_swz(int r) { return (r >> 1) & 7; }
 
 constexpr int MID_BK = 64;     // K elements of a step: 128 bytes of a row
 constexpr int MID_STAGES = 6;  // LDS stages of token rows
-constexpr int MID_RING = 4;    // register sets of weights
 constexpr int MID_LEAD = 4;    // LDS reads ahead of their MFMAs
 
 struct MidArgs {
@@ -97,7 +101,11 @@ struct MidArgs {
 template <int MB>
 constexpr int MID_LOADERS = MB > 4 ? (MB % 2 ? 2 : 4) : MB > 1 ? 2 : 1;
 
-template <int MB, int NB, int NW>
+// Register sets of weights: four steps; three where four would not fit.
+constexpr int mid_ring(int MB, int NB, bool NT) { return NT && MB * NB >= 16 ? 3 : 4; }
+
+// NT: whole-line, non-temporal weight loads.
+template <int MB, int NB, int NW, bool NT>
 __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(MidArgs a) {
     constexpr int LW = MID_LOADERS<MB>, PER = 2 * MB / LW, XT = 16 * MB * 128;  // XT: bytes of a stage
     constexpr int AHEAD = MID_STAGES - 1;
@@ -152,17 +160,39 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
 
     const int g = lane >> 4, n = lane & 15;
     const int row0 = n0 + wave * 16 * NB;
-    const bf16_t* wr[NB];
+    // Load h of block i: with NT whole lines, lane (g, n) chunk g + 4 (n / 8) of
+    // row 16i + 8h + n % 8; else the operand itself, chunk 4h + g of row
+    // 16i + n.  Rows past N re-read the last row.
+    constexpr int RING = mid_ring(MB, NB, NT);
+    const char* wb = reinterpret_cast<const char*>(a.w + (int64_t)row0 * a.K + kb);
+    int woff[NB][2];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) wr[i] = a.w + (int64_t)min(row0 + 16 * i + n, a.N - 1) * a.K + kb + 8 * g;
-    u32x4_t wv[MID_RING][NB][2];
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int row = row0 + 16 * i + (NT ? 8 * h + (n & 7) : n), chunk = NT ? g + 4 * (n >> 3) : 4 * h + g;
+            woff[i][h] = 2 * ((min(row, a.N - 1) - row0) * a.K + 8 * chunk);
+        }
+    u32x4_t wv[RING][NB][2];
     auto load = [&](int c, u32x4_t (&d)[NB][2]) {
-        const int k = min(c, nk - 1) * MID_BK;
+        const char* wc = wb + min(c, nk - 1) * MID_BK * 2;
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
-            for (int kk = 0; kk < 2; ++kk)
-                d[i][kk] = *reinterpret_cast<const u32x4_t*>(wr[i] + k + 32 * kk);
+            for (int h = 0; h < 2; ++h) {
+                const u32x4_t* p = reinterpret_cast<const u32x4_t*>(wc + woff[i][h]);
+                d[i][h] = NT ? __builtin_nontemporal_load(p) : *p;
+            }
+    };
+    // The A operands of a block's two k halves (row n, chunk 4kk + g) from its
+    // two whole-line loads: lanes n >= 8 of the first change places with lanes
+    // n < 8 of the second, eight lanes away in the row of 16.
+    auto operands = [&](const u32x4_t (&d)[2], u32x4_t (&op)[2]) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            op[0][e] = NT ? __builtin_amdgcn_update_dpp(d[0][e], d[1][e], 0x128, 0xf, 0xc, false) : d[0][e];  // row_ror:8
+            op[1][e] = NT ? __builtin_amdgcn_update_dpp(d[1][e], d[0][e], 0x128, 0xf, 0x3, false) : d[1][e];
+        }
     };
     f32x4_t acc[NB][MB];
 #pragma unroll
@@ -175,7 +205,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     for (int kk = 0; kk < 2; ++kk) boff[kk] = (n * 8 + ((4 * kk + g) ^ wide_swz(n))) * 16;
 
 #pragma unroll
-    for (int c = 0; c < MID_RING - 1; ++c) load(c, wv[c]);
+    for (int c = 0; c < RING - 1; ++c) load(c, wv[c]);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     // LDS reads run MID_LEAD operands ahead of their MFMAs; the compiler's own
@@ -184,6 +214,9 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     constexpr int LEAD = MB < MID_LEAD ? MB : MID_LEAD;
     auto step = [&](int c, int u) {
         const char* xp = lds + (c % MID_STAGES) * XT;
+        u32x4_t op[NB][2];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) operands(wv[u][i], op[i]);
         u32x4_t b[2][MB];
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
@@ -194,7 +227,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
 #pragma unroll
             for (int j = 0; j < MB; ++j)
 #pragma unroll
-                for (int i = 0; i < NB; ++i) acc[i][j] = mfma(wv[u][i][kk], b[kk][j], acc[i][j]);
+                for (int i = 0; i < NB; ++i) acc[i][j] = mfma(op[i][kk], b[kk][j], acc[i][j]);
         __builtin_amdgcn_sched_group_barrier(0x100, LEAD, 0);  // LDS reads
 #pragma unroll
         for (int q = 0; q < 2 * MB - LEAD; ++q) {
@@ -204,13 +237,13 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
         __builtin_amdgcn_sched_group_barrier(0x008, LEAD * NB, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    // Groups of MID_RING steps, each step first loading the one MID_RING - 1
-    // ahead; the last group (1..MID_RING steps) has its steps in flight but one.
+    // Groups of RING steps, each step first loading the one RING - 1
+    // ahead; the last group (1..RING steps) has its steps in flight but one.
     int c0 = 0;
-    for (; nk - c0 > MID_RING; c0 += MID_RING) {
+    for (; nk - c0 > RING; c0 += RING) {
 #pragma unroll
-        for (int u = 0; u < MID_RING; ++u) {
-            load(c0 + u + MID_RING - 1, wv[(u + MID_RING - 1) % MID_RING]);
+        for (int u = 0; u < RING; ++u) {
+            load(c0 + u + RING - 1, wv[(u + RING - 1) % RING]);
             // Keep the prefetch here: the scheduler would otherwise sink each
             // load down to its use and the MFMAs would wait for fresh loads.
             __builtin_amdgcn_sched_barrier(0);
@@ -218,10 +251,10 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
             __syncthreads();
         }
     }
-    load(c0 + MID_RING - 1, wv[MID_RING - 1]);
+    load(c0 + RING - 1, wv[RING - 1]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < MID_RING; ++u) {
+    for (int u = 0; u < RING; ++u) {
         if (c0 + u < nk) step(c0 + u, u);
         if (c0 + u + 1 < nk) __syncthreads();
     }
@@ -286,7 +319,8 @@ constexpr int MID_MIN_SPLIT_STEPS = 4;  // K steps of a split, at least
 // arithmetic, so a step costs about 20 ns per 16-row block that the workgroup
 // loads (weights or tokens) plus 100 ns of barrier and latency, once per round
 // of workgroups over the CUs; splitting adds its partials' traffic (write and
-// read at 5 TB/s) and the reduce launch (4.5 us).  Against a sweep of all
+// read at 4 TB/s) and the reduce launch (6 us with its start-up; o at 200
+// tokens 17.5 us split in four, 15.8 whole; at 33 tokens 10.0 in eight, 12.8).  Against a sweep of all
 // shapes at 12-1000 tokens on the four projections the pick is the fastest or
 // within 8% of it (o at 512 tokens 26.0 against 23.8 us at worst).  With
 // fixed_splits, the best tile for that many splits.
@@ -310,7 +344,7 @@ inline MidPlan mid_plan(int M, int N, int K, int cus, int max_splits, int fixed_
             // Splits only within one round of workgroups.
             for (int s = 1; s == 1 || (s <= max_splits && tiles * s <= cus && steps >= s * MID_MIN_SPLIT_STEPS); ++s) {
                 double us = 0.02 * (5 + wb + mb) * ((steps + s - 1) / s) * rounds;
-                if (s > 1) us += 4.5 + (double)s * M * N * 8.0 / 5e6;
+                if (s > 1) us += 6.0 + (double)s * M * N * 8.0 / 4e6;
                 if (us < best_us) {
                     best_us = us;
                     best = {mb, sh[0], sh[1], s};
@@ -327,7 +361,10 @@ int launch_mid_mb(const MidPlan& p, const MidArgs& a, hipStream_t stream) {
     switch (p.nb * 10 + p.nw) {
 #define Q3_MID(nb, nw)                                                                                           \
     case nb * 10 + nw:                                                                                           \
-        Q3_LAUNCH((gemm_mid_kernel<MB, nb, nw>), grid, dim3((nw + MID_LOADERS<MB>) * 64), 0, stream, a);         \
+        if (a.tm == 1)                                                                                           \
+            Q3_LAUNCH((gemm_mid_kernel<MB, nb, nw, true>), grid, dim3((nw + MID_LOADERS<MB>) * 64), 0, stream, a); \
+        else                                                                                                     \
+            Q3_LAUNCH((gemm_mid_kernel<MB, nb, nw, false>), grid, dim3((nw + MID_LOADERS<MB>) * 64), 0, stream, a); \
         return (int)hipGetLastError();
         Q3_MID(1, 2) Q3_MID(1, 3) Q3_MID(1, 4) Q3_MID(1, 5) Q3_MID(2, 3) Q3_MID(2, 5) Q3_MID(2, 8)
 #undef Q3_MID

@@ -334,11 +334,6 @@ class Engine:
             for N, K in self._projections():
                 ws = max(ws, call("q3_skinny_splits", B, N, K) * B * N)
         self.skinny_ws = self._empty(max(ws, 1), dtype=torch.float32)
-        # Split partials of the other MFMA decode projections (more than 64 rows).
-        ws = 0
-        if not self.small and not self.skinny:
-            ws = max(call("q3_gemm_ws_floats", B, N, K) for N, K in self._projections())
-        self.proj_ws = self._empty(max(ws, 1), dtype=torch.float32)
         if self.small:
             self.lm_parts = call("q3_gemv_partials", B, V, _lib.EPI_ARGMAX)
         elif self.skinny:
@@ -551,9 +546,8 @@ class Engine:
 
     def _proj(self, x: int, ldx: int, w: torch.Tensor, N: int, K: int, epi: int, y: int, ldy: int) -> None:
         """Decode projection for batches outside the GEMV and fused MFMA paths (more
-        than 64 rows, or shapes that do not tile): the short-prompt MFMA GEMM,
-        long K split over workgroups (down at 100 rows: 30.5 us unsplit, 18.8 split)."""
-        call("q3_gemm_ws", x, ldx, _ptr(w), self.batch, N, K, epi, y, ldy, _ptr(self.proj_ws), self._s)
+        than 64 rows, or shapes that do not tile): the short-prompt MFMA GEMM."""
+        call("q3_gemm", x, ldx, _ptr(w), self.batch, N, K, epi, y, ldy, self._s)
 
     def _capture(self) -> None:
         """Warm every kernel eagerly, then record one decode step as a hipGraph.
@@ -646,14 +640,6 @@ class Engine:
             self._prefill_part = self._empty(floats, dtype=torch.float32)
         return self._prefill_part
 
-    def _residual_splits(self, M: int, K: int) -> int:
-        """K splits of a residual projection over M prompt tokens whose partials
-        the residual add + RMSNorm sums; 0 where it is not split."""
-        s = call("q3_gemm_splits", M, self.HIDDEN, K)
-        if not s and M < 256:  # the short-prompt tiling's own count
-            s = call("q3_gemm_ws_floats", M, self.HIDDEN, K) // (M * self.HIDDEN)
-        return s
-
     def _forward_prefill(self, ids: torch.Tensor, seq_len: int) -> torch.Tensor:
         """Consume the prompt ``ids [B, P]``; return the last position's logits [B, 1, V].
 
@@ -695,12 +681,16 @@ class Engine:
                 # residual projections along K; their partials are summed (in split
                 # order), joined to the residual and normalised by one row kernel,
                 # which replaces the RMSNorm that follows each of them.
-                s_o, s_d = self._residual_splits(M, self.q_size), self._residual_splits(M, I)
+                s_o = call("q3_gemm_splits", M, H, self.q_size)
+                s_d = call("q3_gemm_splits", M, H, I)
                 # Longer prompts whose last round of tiles is at most half full split
                 # those tiles along K (q3_gemm_ws); the same buffer holds either.
+                # Below 256 tokens no workspace, so nothing is split: the same sums in
+                # the same order whatever the row count, hence the same tokens.
                 floats = max(s_o, s_d) * M * H
                 for n_, k_ in ((self.qkv_size, H), (2 * I, H), (H, self.q_size), (H, I)):
-                    floats = max(floats, call("q3_gemm_ws_floats", M, n_, k_))
+                    if M >= 256:
+                        floats = max(floats, call("q3_gemm_ws_floats", M, n_, k_))
                 part = _ptr(self._prefill_partials(floats)) if floats else None
                 for i, L in enumerate(self.layers):
                     if i == 0:
