@@ -104,8 +104,8 @@ int q3_gemm_partials(const uint16_t *x, int ldx, const uint16_t *w, int M, int N
  * the other tiles are q3_gemm's, bit for bit.  Below 256 tokens, projections
  * of long K may split K over all tiles the same way.  ws holds
  * q3_gemm_ws_floats(M, N, K) floats (0: nothing is split, and q3_gemm_ws is
- * q3_gemm), 16-byte aligned; below 256 tokens ws may be NULL (nothing is
- * split).  Same operand rules as q3_gemm. */
+ * q3_gemm), 16-byte aligned; below 256 tokens ws may be NULL or unaligned
+ * (nothing is split).  Same operand rules as q3_gemm. */
 int q3_gemm_ws_floats(int M, int N, int K);
 int q3_gemm_ws(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
                int epi, uint16_t *y, int ldy, float *ws, hipStream_t stream);

@@ -465,8 +465,9 @@ extern "C" int q3_gemm_ws_floats(int M, int N, int K) {
 extern "C" int q3_gemm_ws(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y,
                           int ldy, float* ws, hipStream_t stream) {
     const int need = q3_gemm_ws_floats(M, N, K);
-    if (need == 0 || epi == EPI_PARTIAL || (M < 256 && !ws)) return q3_gemm(x, ldx, w, M, N, K, epi, y, ldy, stream);
-    if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15)) return (int)hipErrorInvalidValue;
+    const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
+    if (need == 0 || epi == EPI_PARTIAL || (M < 256 && !ws_ok)) return q3_gemm(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    if (!ws_ok) return (int)hipErrorInvalidValue;
     // The operand checks of q3_gemm.
     if (N % 4 || ldx % 8 || ldx < K || ldy % 4 || !x || !w || !y ||
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) ||

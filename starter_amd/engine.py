@@ -653,7 +653,7 @@ class Engine:
                              f"(batch {self.batch}, capacity {self.capacity})")
         # One reduction and one copy back for both bounds (ids on the device
         # would take two of each, with the GPU idle meanwhile).
-        lo, hi = torch.stack(torch.aminmax(ids)).tolist()
+        lo, hi = map(int, torch.stack(torch.aminmax(ids)).tolist())
         if lo < 0 or hi >= self.VOCAB:
             raise ValueError(f"token ids must lie in [0, {self.VOCAB})")
         if ids.is_cuda:

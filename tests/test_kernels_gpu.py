@@ -422,6 +422,13 @@ def test_gemm_short_prompt_tiles(M, N, K):
                   *tail)
         assert_nearly_exact(act, oc.swiglu(y[:, 0::2], y[:, 1::2]), frac=5e-3)
     assert torch.all(ws.cpu()[floats:] == 9.0)
+    # Without a usable workspace nothing is split: q3_gemm, bit for bit, and no byte of ws touched.
+    if M < 256:
+        fill = torch.full((M + 2, ld(N)), 5.0, dtype=torch.bfloat16)
+        whole, before = run("q3_gemm", _lib.EPI_STORE, N, fill), ws.cpu()
+        for ptr in (None, P(ws) + 4):
+            assert torch.equal(run("q3_gemm_ws", _lib.EPI_STORE, N, fill, ptr), whole)
+        assert torch.equal(ws.cpu(), before)
 
 
 @pytest.mark.parametrize("M,N,K,epi", [(4096, 6144, 2560, _lib.EPI_STORE), (4096, 2560, 4096, _lib.EPI_RESID),
