@@ -6,7 +6,7 @@
 // far outweigh the arithmetic, so the kernel is built around two streams that
 // never wait for each other:
 //   * weights go from HBM (row-major, 128 bytes of a row per step of 64 K)
-//     straight into MFMA A operands, two or three steps ahead in registers;
+//     straight into MFMA A operands, two to seven steps ahead in registers;
 //     each weight row is read by one wave, which holds 16 * NB of them.  An
 //     operand is 64 bytes of 16 rows.  With one token tile each weight is read
 //     once: a load instruction then takes whole 128-byte lines of eight rows,
@@ -18,7 +18,7 @@
 //     non-temporal half lines 26.3, plain half lines 20.6, whole lines 18.2; at
 //     100 tokens 35.3 / 30.7 / 27.1);
 //   * the 16 * MB token rows of a step are filled into LDS by loader waves
-//     with direct global-to-LDS loads, MID_STAGES - 1 steps ahead, and feed
+//     with direct global-to-LDS loads, STAGES - 1 steps ahead, and feed
 //     every compute wave as B operands.  Waves of their own, because vector
 //     memory counters retire in order: a compute wave that loaded both would
 //     wait for its newest token rows with every weight it needs.  One wave
@@ -80,7 +80,6 @@ __device__ __forceinline__ void store4(bf16_t* y, int ldy, int m, int col, const
 __device__ __forceinline__ int wide_swz(int r) { return (r >> 1) & 7; }
 
 constexpr int MID_BK = 64;     // K elements of a step: 128 bytes of a row
-constexpr int MID_STAGES = 6;  // LDS stages of token rows
 constexpr int MID_LEAD = 4;    // LDS reads ahead of their MFMAs
 
 struct MidArgs {
@@ -101,16 +100,33 @@ struct MidArgs {
 template <int MB>
 constexpr int MID_LOADERS = MB > 4 ? (MB % 2 ? 2 : 4) : MB > 1 ? 2 : 1;
 
-// Register sets of weights: four steps; three where four would not fit.
-constexpr int mid_ring(int MB, int NB, bool NT) { return NT && MB * NB >= 16 ? 3 : 4; }
+// Two compute waves of 16 rows keep too few bytes in flight with three steps
+// ahead: at 0.6 us of latency a step took 0.2 us whatever the token count.
+// Seven ahead (us, three -> seven: o at 9 / 45 / 80 / 128 tokens 14.2 / 13.5 /
+// 14.1 / 15.0 -> 10.4 / 11.2 / 12.3 / 14.5; down 30.9 / 28.7 / 29.8 / 31.7 ->
+// 21.7 / 23.4 / 25.9 / 30.9; qkv at 9 / 33 tokens 10.8 / 11.6 -> 8.5 / 11.1).
+// Wider workgroups are no faster so, or slower (qkv in three waves at 80 tokens
+// 14.1 -> 14.5, gate/up in five at 128 34.8 -> 41.5, down in eight splits at 45
+// 15.7 -> 16.8), nor are two waves beside five or more token blocks (o at 200
+// tokens 17.6 -> 17.7).
+constexpr bool mid_deep(int MB, int NB, int NW) { return NB == 1 && NW == 2 && MB <= 4; }
+
+// LDS stages of token rows.
+constexpr int mid_stages(int MB, int NB, int NW) { return mid_deep(MB, NB, NW) ? 8 : 6; }
+
+// Register sets of weights, one more than the steps ahead; three where four
+// would not fit.
+constexpr int mid_ring(int MB, int NB, int NW, bool NT) {
+    return mid_deep(MB, NB, NW) ? 8 : NT && MB * NB >= 16 ? 3 : 4;
+}
 
 // NT: whole-line, non-temporal weight loads.
 template <int MB, int NB, int NW, bool NT>
 __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(MidArgs a) {
     constexpr int LW = MID_LOADERS<MB>, PER = 2 * MB / LW, XT = 16 * MB * 128;  // XT: bytes of a stage
-    constexpr int AHEAD = MID_STAGES - 1;
+    constexpr int STAGES = mid_stages(MB, NB, NW), AHEAD = STAGES - 1;
     static_assert(2 * MB % LW == 0 && PER * AHEAD <= 63, "direct loads in flight exceed the vmcnt range");
-    __shared__ __align__(1024) char lds[MID_STAGES * XT];
+    __shared__ __align__(1024) char lds[STAGES * XT];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
@@ -139,7 +155,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
         const uint32_t lbase = lds_address(lds) + 1024 * lw;
         auto issue = [&](int c) {
             const bf16_t* xc = xb + min(c, nk - 1) * MID_BK;
-            const uint32_t sbase = lbase + (uint32_t)(c % MID_STAGES) * XT;
+            const uint32_t sbase = lbase + (uint32_t)(c % STAGES) * XT;
 #pragma unroll
             for (int i = 0; i < PER; ++i) load_to_lds(xc, voff[i], sbase + 1024 * LW * i);
         };
@@ -148,7 +164,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
         wait_vmcnt<PER * (AHEAD - 1)>();
         __syncthreads();
         for (int c = 0; c + 1 < nk; ++c) {
-            // Stage (c + AHEAD) % MID_STAGES was last read in step c - 1, which
+            // Stage (c + AHEAD) % STAGES was last read in step c - 1, which
             // every wave finished before the barrier that ended it.
             issue(c + AHEAD);
             wait_vmcnt<PER * (AHEAD - 1)>();  // step c + 1 landed
@@ -163,7 +179,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     // Load h of block i: with NT whole lines, lane (g, n) chunk g + 4 (n / 8) of
     // row 16i + 8h + n % 8; else the operand itself, chunk 4h + g of row
     // 16i + n.  Rows past N re-read the last row.
-    constexpr int RING = mid_ring(MB, NB, NT);
+    constexpr int RING = mid_ring(MB, NB, NW, NT);
     const char* wb = reinterpret_cast<const char*>(a.w + (int64_t)row0 * a.K + kb);
     int woff[NB][2];
 #pragma unroll
@@ -213,7 +229,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     // 30.7 us).
     constexpr int LEAD = MB < MID_LEAD ? MB : MID_LEAD;
     auto step = [&](int c, int u) {
-        const char* xp = lds + (c % MID_STAGES) * XT;
+        const char* xp = lds + (c % STAGES) * XT;
         u32x4_t op[NB][2];
 #pragma unroll
         for (int i = 0; i < NB; ++i) operands(wv[u][i], op[i]);

@@ -385,10 +385,11 @@ def test_gemm(M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 32, 64), (15, 36, 192), (16, 2560, 4096), (17, 2560, 9728), (33, 260, 320),
                                    (45, 2560, 9728), (81, 84, 576), (127, 6144, 2560), (128, 2560, 9728),
-                                   (129, 1028, 832), (255, 2560, 4096), (257, 3800, 448), (511, 516, 64)])
+                                   (129, 1028, 832), (255, 2560, 4096), (257, 3800, 448), (511, 516, 64),
+                                   (40, 100, 512), (61, 68, 576), (64, 2556, 1088)])
 def test_gemm_short_prompt_tiles(M, N, K):
     """The loader-wave tiling of q3_gemm / q3_gemm_ws below the 256 x 256 one: token and weight tiles that end
-    inside a 16-row block, one K step up to more than a register ring, splits with uneven K ranges (the 2560-wide
+    inside a 16-row block, one K step up to one and two more than a register ring and its multiples, splits with uneven K ranges (the 2560-wide
     long-K shapes).  Sampled rows against float64; nothing written past N or M; both epilogues of the split path
     bit-exact against its own stored projection."""
     assert call("q3_gemm_tiles_wide", M, N) == 0
