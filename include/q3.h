@@ -101,11 +101,10 @@ int q3_gemm_partials(const uint16_t *x, int ldx, const uint16_t *w, int M, int N
  * full -- or, at 256+ tokens below q3_gemm_tiles_wide, where all the tiles
  * fill at most half the CUs -- those tiles are split along K and a second
  * kernel sums their FP32 partials in split order and applies the epilogue;
- * the other tiles are q3_gemm's, bit for bit.  Below 256 tokens, projections
- * of long K may split K over all tiles the same way.  ws holds
- * q3_gemm_ws_floats(M, N, K) floats (0: nothing is split, and q3_gemm_ws is
- * q3_gemm), 16-byte aligned; below 256 tokens ws may be NULL or unaligned
- * (nothing is split).  Same operand rules as q3_gemm. */
+ * the other tiles are q3_gemm's, bit for bit.  ws holds
+ * q3_gemm_ws_floats(M, N, K) floats, 16-byte aligned; where that is 0, as
+ * always below 256 tokens, nothing is split, q3_gemm_ws is q3_gemm, and ws is
+ * neither read nor written.  Same operand rules as q3_gemm. */
 int q3_gemm_ws_floats(int M, int N, int K);
 int q3_gemm_ws(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
                int epi, uint16_t *y, int ldy, float *ws, hipStream_t stream);

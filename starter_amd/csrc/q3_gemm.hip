@@ -420,7 +420,7 @@ extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, 
     if (q3_gemm_tiles_wide(M, N))
         return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, ((M + 255) / 256) * ((N + 255) / 256), 1, nullptr,
                            stream);
-    return launch_mid(mid_plan(M, N, K, mid_cus(), 1), x, ldx, w, M, N, K, epi, y, ldy, nullptr, stream);
+    return launch_mid(mid_plan(M, N, mid_cus()), x, ldx, w, M, N, K, epi, y, ldy, nullptr, stream);
 }
 
 // Split tail of the wide tiling.  One 256 x 256-tile workgroup fits a CU
@@ -453,11 +453,6 @@ static WidePlan wide_tail_plan(int M, int N, int K) {
 
 extern "C" int q3_gemm_ws_floats(int M, int N, int K) {
     if (M < 1 || N < 4 || K < WIDE_BK || K % WIDE_BK) return 0;
-    if (M < 256) {
-        const MidPlan p = mid_plan(M, N, K, mid_cus(), MID_MAX_SPLITS);
-        const int64_t floats = p.splits > 1 ? (int64_t)p.splits * M * N : 0;
-        return floats <= INT32_MAX ? (int)floats : 0;
-    }
     const WidePlan p = wide_tail_plan(M, N, K);
     return p.tail * p.splits * 256 * 256;
 }
@@ -465,17 +460,14 @@ extern "C" int q3_gemm_ws_floats(int M, int N, int K) {
 extern "C" int q3_gemm_ws(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y,
                           int ldy, float* ws, hipStream_t stream) {
     const int need = q3_gemm_ws_floats(M, N, K);
-    const bool ws_ok = ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
-    if (need == 0 || epi == EPI_PARTIAL || (M < 256 && !ws_ok)) return q3_gemm(x, ldx, w, M, N, K, epi, y, ldy, stream);
-    if (!ws_ok) return (int)hipErrorInvalidValue;
+    if (need == 0 || epi == EPI_PARTIAL) return q3_gemm(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15)) return (int)hipErrorInvalidValue;
     // The operand checks of q3_gemm.
     if (N % 4 || ldx % 8 || ldx < K || ldy % 4 || !x || !w || !y ||
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) ||
         (reinterpret_cast<uintptr_t>(y) & 7))
         return (int)hipErrorInvalidValue;
     if ((int64_t)256 * ldx * 2 > INT32_MAX || (int64_t)256 * K * 2 > INT32_MAX) return (int)hipErrorInvalidValue;
-    if (M < 256)  // need > 0: the plan splits K
-        return launch_mid(mid_plan(M, N, K, mid_cus(), MID_MAX_SPLITS), x, ldx, w, M, N, K, epi, y, ldy, ws, stream);
     const WidePlan p = wide_tail_plan(M, N, K);
     return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, p.full, p.splits, ws, stream);
 }
@@ -515,7 +507,7 @@ extern "C" int q3_gemm_partials(const bf16_t* x, int ldx, const bf16_t* w, int M
     // Below one token tile the mid tiling (o / down at 100 tokens, 8 splits:
     // 8.4 / 15.0 us; a 256-token tile would be mostly empty).
     if (M < 256)
-        return launch_mid(mid_plan(M, N, K, mid_cus(), splits, splits), x, ldx, w, M, N, K, EPI_PARTIAL, nullptr, 0,
-                          ws, stream);
+        return launch_mid(mid_plan(M, N, mid_cus(), splits), x, ldx, w, M, N, K, EPI_PARTIAL, nullptr, 0, ws,
+                          stream);
     return launch_wide(x, ldx, w, M, N, K, EPI_PARTIAL, nullptr, 0, 0, splits, ws, stream);
 }

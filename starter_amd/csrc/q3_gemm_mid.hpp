@@ -25,9 +25,8 @@
 //     streams at most ~27 GB/s whatever its depth, four ~100 GB/s, hence the
 //     loader counts (gate/up at 250 tokens: two loaders 57 us, four 45).
 // A workgroup is NW compute waves (16 NB NW weight rows) and the loader waves,
-// one barrier per step; with split > 1 the workgroups of a tile take
-// contiguous K ranges and mid_reduce_kernel sums their FP32 partials in split
-// order and applies the epilogue.
+// one barrier per step; with splits > 1 the workgroups of a tile take
+// contiguous K ranges and store FP32 partials (EPI_PARTIAL).
 //
 // What bounds it: the weights' HBM stream (5.5 TB/s at 16 tokens on gate/up,
 // launch included) and, from ~64 tokens on, the token rows beside it: without
@@ -296,30 +295,6 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     }
 }
 
-// Sum of the split partials in split order, then the epilogue; thread: four
-// columns of one token row.  Every split's load is issued before the sum.
-constexpr int MID_MAX_SPLITS = 8;
-
-template <int EPI>
-__global__ __launch_bounds__(256) void mid_reduce_kernel(const float* __restrict__ part, int splits, int M, int N,
-                                                         bf16_t* y, int ldy) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int quads = N / 4;
-    if (e >= (int64_t)M * quads) return;
-    const int m = (int)(e / quads), c = 4 * (int)(e % quads);
-    const float* src = part + (int64_t)m * N + c;
-    const int64_t stride = (int64_t)M * N;
-    f32x4_t p[MID_MAX_SPLITS];
-#pragma unroll
-    for (int s = 0; s < MID_MAX_SPLITS; ++s)
-        p[s] = *reinterpret_cast<const f32x4_t*>(src + min(s, splits - 1) * stride);
-    f32x4_t v = p[0];
-#pragma unroll
-    for (int s = 1; s < MID_MAX_SPLITS; ++s)
-        if (s < splits) v += p[s];
-    store4<EPI>(y, ldy, m, c, v);
-}
-
 // Launch shape: MB token blocks x NB NW weight blocks of 16 per workgroup, and
 // the K splits.
 struct MidPlan {
@@ -329,42 +304,23 @@ struct MidPlan {
 // The tile shapes that are built, as NB, NW.
 constexpr int MID_SHAPES[][2] = {{1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 3}, {2, 5}, {2, 8}};
 constexpr int MID_MAX_MB = 8;
-constexpr int MID_MIN_SPLIT_STEPS = 4;  // K steps of a split, at least
 
 // Picks the plan of least estimated time.  A CU's bytes set it, not its
 // arithmetic, so a step costs about 20 ns per 16-row block that the workgroup
 // loads (weights or tokens) plus 100 ns of barrier and latency, once per round
-// of workgroups over the CUs; splitting adds its partials' traffic (write and
-// read at 4 TB/s) and the reduce launch (6 us with its start-up; o at 200
-// tokens 17.5 us split in four, 15.8 whole; at 33 tokens 10.0 in eight, 12.8).  Against a sweep of all
-// shapes at 12-1000 tokens on the four projections the pick is the fastest or
-// within 8% of it (o at 512 tokens 26.0 against 23.8 us at worst).  With
-// fixed_splits, the best tile for that many splits.
-inline MidPlan mid_plan(int M, int N, int K, int cus, int max_splits, int fixed_splits = 0) {
-    const int steps = K / MID_BK, mblocks = (M + 15) / 16, nblocks = (N + 15) / 16;
-    MidPlan best{1, 1, 2, fixed_splits ? fixed_splits : 1};
-    double best_us = 1e30;
+// of workgroups over the CUs.
+inline MidPlan mid_plan(int M, int N, int cus, int splits = 1) {
+    const int mblocks = (M + 15) / 16, nblocks = (N + 15) / 16;
+    MidPlan best{1, 1, 2, splits};
+    double best_cost = 1e30;
     for (const auto& sh : MID_SHAPES) {
         const int wb = sh[0] * sh[1];
         for (int mb = mblocks < MID_MAX_MB ? mblocks : MID_MAX_MB; mb >= 1; --mb) {
             const int64_t tiles = (int64_t)((mblocks + mb - 1) / mb) * ((nblocks + wb - 1) / wb);
-            if (fixed_splits) {
-                const double us = 0.02 * (5 + wb + mb) * (double)((tiles * fixed_splits + cus - 1) / cus);
-                if (us < best_us) {
-                    best_us = us;
-                    best = {mb, sh[0], sh[1], fixed_splits};
-                }
-                continue;
-            }
-            const double rounds = (double)((tiles + cus - 1) / cus);
-            // Splits only within one round of workgroups.
-            for (int s = 1; s == 1 || (s <= max_splits && tiles * s <= cus && steps >= s * MID_MIN_SPLIT_STEPS); ++s) {
-                double us = 0.02 * (5 + wb + mb) * ((steps + s - 1) / s) * rounds;
-                if (s > 1) us += 6.0 + (double)s * M * N * 8.0 / 4e6;
-                if (us < best_us) {
-                    best_us = us;
-                    best = {mb, sh[0], sh[1], s};
-                }
+            const double cost = (5 + wb + mb) * (double)((tiles * splits + cus - 1) / cus);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = {mb, sh[0], sh[1], splits};
             }
         }
     }
@@ -388,18 +344,17 @@ int launch_mid_mb(const MidPlan& p, const MidArgs& a, hipStream_t stream) {
     return (int)hipErrorInvalidValue;
 }
 
-// y = epi(x . W^T) under plan p; part holds [p.splits, M, N] floats when
-// p.splits > 1 or epi is EPI_PARTIAL (which leaves the sum to the caller).
+// y = epi(x . W^T) under plan p, or with EPI_PARTIAL its K-split partials to
+// part [p.splits, M, N].
 inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi,
                       bf16_t* y, int ldy, float* part, hipStream_t stream) {
     const bool partial = epi == EPI_PARTIAL;
     if (!partial && epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU)
         return (int)hipErrorInvalidValue;
-    if ((p.splits > 1 || partial) && !part) return (int)hipErrorInvalidValue;
-    if (p.splits > MID_MAX_SPLITS && !partial) return (int)hipErrorInvalidValue;
+    if (partial != (part != nullptr) || (p.splits > 1 && !partial)) return (int)hipErrorInvalidValue;
     const int tm = (M + 16 * p.mb - 1) / (16 * p.mb), tn = (N + 16 * p.nb * p.nw - 1) / (16 * p.nb * p.nw);
     if ((int64_t)tm * tn * p.splits > (1 << 30)) return (int)hipErrorInvalidValue;
-    const MidArgs a{x, ldx, w, M, N, K, p.splits > 1 ? EPI_PARTIAL : epi, y, ldy, part, tm, tn, p.splits};
+    const MidArgs a{x, ldx, w, M, N, K, epi, y, ldy, part, tm, tn, p.splits};
     int rc = (int)hipErrorInvalidValue;
     switch (p.mb) {
         case 1: rc = launch_mid_mb<1>(p, a, stream); break;
@@ -411,15 +366,7 @@ inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* 
         case 7: rc = launch_mid_mb<7>(p, a, stream); break;
         case 8: rc = launch_mid_mb<8>(p, a, stream); break;
     }
-    if (rc || partial || p.splits == 1) return rc;
-    const dim3 grid((unsigned)(((int64_t)M * (N / 4) + 255) / 256));
-    if (epi == Q3_EPI_SWIGLU)
-        Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_SWIGLU>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);
-    else if (epi == Q3_EPI_RESID)
-        Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_RESID>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);
-    else
-        Q3_LAUNCH(mid_reduce_kernel<Q3_EPI_STORE>, grid, dim3(256), 0, stream, part, p.splits, M, N, y, ldy);
-    Q3_CHECK_LAUNCH();
+    return rc;
 }
 
 }  // namespace q3gemm

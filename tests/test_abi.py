@@ -118,3 +118,11 @@ def test_prompt_gemm_split_policy():
     assert _lib.call("q3_gemm_splits", 700, 3800, 576) == 2
     with pytest.raises(RuntimeError, match="q3_gemm_partials failed"):
         _lib.call("q3_gemm_partials", None, 4096, None, 1024, H, 4096, None, 17, None)  # > 16 splits
+
+
+def test_gemm_ws_below_256_tokens_needs_no_workspace():
+    """Below 256 tokens q3_gemm_ws splits nothing: its sums keep q3_gemm's order at every row count, and a buffer that
+    was sized for longer prompts only is never written."""
+    for N, K in ((6144, 2560), (2560, 4096), (19456, 2560), (2560, 9728), (512, 8192), (64, 64)):
+        for M in (1, 9, 45, 100, 200, 255):
+            assert _lib.call("q3_gemm_ws_floats", M, N, K) == 0, (M, N, K)

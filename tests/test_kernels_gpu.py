@@ -389,14 +389,14 @@ def test_gemm(M, N, K):
                                    (40, 100, 512), (61, 68, 576), (64, 2556, 1088)])
 def test_gemm_short_prompt_tiles(M, N, K):
     """The loader-wave tiling of q3_gemm / q3_gemm_ws below the 256 x 256 one: token and weight tiles that end
-    inside a 16-row block, one K step up to one and two more than a register ring and its multiples, splits with uneven K ranges (the 2560-wide
-    long-K shapes).  Sampled rows against float64; nothing written past N or M; both epilogues of the split path
-    bit-exact against its own stored projection."""
+    inside a 16-row block, one K step up to one and two more than a register ring and its multiples.  Sampled rows
+    against float64; nothing written past N or M; the residual join bit-exact against the stored projection.  Below 256
+    tokens q3_gemm_ws is q3_gemm, bit for bit, whatever its workspace, of which it touches no byte."""
     assert call("q3_gemm_tiles_wide", M, N) == 0
     x, w = rnd((M, K), 1.0, M + 61), rnd((N, K), 0.02, N + K + 61)
     xd, wd = dv(x), dv(w)
     floats = call("q3_gemm_ws_floats", M, N, K)
-    assert floats > 0 or (N, K) != (2560, 9728)  # the down projection's shape splits K
+    assert floats == 0 or M >= 256
     ws = dv(torch.full((floats + 64,), 9.0, dtype=torch.float32))
     g = torch.Generator().manual_seed(M)
     rows = torch.cat([torch.tensor([0, M - 1]), torch.randint(0, M, (30,), generator=g)])
@@ -423,13 +423,12 @@ def test_gemm_short_prompt_tiles(M, N, K):
                   *tail)
         assert_nearly_exact(act, oc.swiglu(y[:, 0::2], y[:, 1::2]), frac=5e-3)
     assert torch.all(ws.cpu()[floats:] == 9.0)
-    # Without a usable workspace nothing is split: q3_gemm, bit for bit, and no byte of ws touched.
     if M < 256:
         fill = torch.full((M + 2, ld(N)), 5.0, dtype=torch.bfloat16)
-        whole, before = run("q3_gemm", _lib.EPI_STORE, N, fill), ws.cpu()
-        for ptr in (None, P(ws) + 4):
+        whole = run("q3_gemm", _lib.EPI_STORE, N, fill)
+        for ptr in (None, P(ws), P(ws) + 4):
             assert torch.equal(run("q3_gemm_ws", _lib.EPI_STORE, N, fill, ptr), whole)
-        assert torch.equal(ws.cpu(), before)
+        assert torch.all(ws.cpu() == 9.0)
 
 
 @pytest.mark.parametrize("M,N,K,epi", [(4096, 6144, 2560, _lib.EPI_STORE), (4096, 2560, 4096, _lib.EPI_RESID),
