@@ -90,9 +90,8 @@ int q3_gemm_tiles_wide(int M, int N);
  * down, engine.py:439,450, at 256-4095 tokens): FP32 partials
  * ws [splits, M, N] (splits * M * N floats), summed in split order by
  * q3_add_rmsnorm_partials.  q3_gemm_splits(M, N, K) is the split count where
- * that applies (else 0); q3_gemm_partials takes any M and any splits in
- * 1..min(16, K / 64) (below 256 tokens on the short-prompt tiling).  Same
- * operand rules as q3_gemm; ws 16-byte aligned. */
+ * that applies (else 0); q3_gemm_partials takes any splits in
+ * 1..min(16, K / 64).  Same operand rules as q3_gemm; ws 16-byte aligned. */
 int q3_gemm_splits(int M, int N, int K);
 int q3_gemm_partials(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,
                      float *ws, int splits, hipStream_t stream);

@@ -121,6 +121,7 @@ constexpr int WIDE_CPR = 8;                          // 16-byte chunks per 128-b
 constexpr int WIDE_TCH = 256 * WIDE_CPR;             // chunks per operand tile
 constexpr int WIDE_DPT = WIDE_TCH / WIDE_THREADS;    // direct loads per operand per thread per step
 constexpr int WIDE_GROUP = 4;                        // token tiles per raster group
+constexpr int EPI_PARTIAL = -1;                      // FP32 split partials, no rounding
 
 // Origin of tile t of a tm x tn grid in raster order: groups of WIDE_GROUP
 // token tiles sweeping the weight tiles (the group's token tiles share each
@@ -420,7 +421,7 @@ extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, 
     if (q3_gemm_tiles_wide(M, N))
         return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, ((M + 255) / 256) * ((N + 255) / 256), 1, nullptr,
                            stream);
-    return launch_mid(mid_plan(M, N, mid_cus()), x, ldx, w, M, N, K, epi, y, ldy, nullptr, stream);
+    return launch_mid(mid_plan(M, N, mid_cus()), x, ldx, w, M, N, K, epi, y, ldy, stream);
 }
 
 // Split tail of the wide tiling.  One 256 x 256-tile workgroup fits a CU
@@ -504,10 +505,5 @@ extern "C" int q3_gemm_partials(const bf16_t* x, int ldx, const bf16_t* w, int M
     if ((int64_t)256 * ldx * 2 > INT32_MAX || (int64_t)256 * K * 2 > INT32_MAX) return (int)hipErrorInvalidValue;
     const int64_t grid = (int64_t)((M + 255) / 256) * ((N + 255) / 256) * splits;
     if (grid > (1 << 30)) return (int)hipErrorInvalidValue;
-    // Below one token tile the mid tiling (o / down at 100 tokens, 8 splits:
-    // 8.4 / 15.0 us; a 256-token tile would be mostly empty).
-    if (M < 256)
-        return launch_mid(mid_plan(M, N, mid_cus(), splits), x, ldx, w, M, N, K, EPI_PARTIAL, nullptr, 0, ws,
-                          stream);
     return launch_wide(x, ldx, w, M, N, K, EPI_PARTIAL, nullptr, 0, 0, splits, ws, stream);
 }

@@ -25,8 +25,7 @@
 //     streams at most ~27 GB/s whatever its depth, four ~100 GB/s, hence the
 //     loader counts (gate/up at 250 tokens: two loaders 57 us, four 45).
 // A workgroup is NW compute waves (16 NB NW weight rows) and the loader waves,
-// one barrier per step; with splits > 1 the workgroups of a tile take
-// contiguous K ranges and store FP32 partials (EPI_PARTIAL).
+// one barrier per step.
 //
 // What bounds it: the weights' HBM stream (5.5 TB/s at 16 tokens on gate/up,
 // launch included) and, from ~64 tokens on, the token rows beside it: without
@@ -45,8 +44,6 @@
 namespace q3gemm {
 
 using namespace q3dma;
-
-constexpr int EPI_PARTIAL = -1;  // FP32 split partials, no rounding
 
 __device__ __forceinline__ f32x4_t mfma(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
@@ -86,12 +83,10 @@ struct MidArgs {
     int ldx;
     const bf16_t* w;
     int M, N, K;
-    int epi;        // Q3_EPI_* or EPI_PARTIAL
+    int epi;
     bf16_t* y;
     int ldy;
-    float* part;    // [splits, M, N] (EPI_PARTIAL)
-    int tm, tn;     // token and weight tiles
-    int splits;
+    int tm;  // token tiles
 };
 
 // Loader waves: one per SIMD where the token rows of a step are most of the
@@ -133,18 +128,15 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     // tiles fastest, so the workgroups that share weight rows share an L2.
     const int total = gridDim.x, xcd = blockIdx.x & 7, q = total >> 3, rem = total & 7;
     const int v = xcd * q + min(xcd, rem) + (int)(blockIdx.x >> 3);
-    const int mt = v % a.tm, nt = (v / a.tm) % a.tn, split = v / (a.tm * a.tn);
-    const int m0 = mt * 16 * MB, n0 = nt * 16 * NB * NW;
-    const int steps = a.K / MID_BK;
-    const int nk = steps / a.splits + (split < steps % a.splits ? 1 : 0);
-    const int kb = (split * (steps / a.splits) + min(split, steps % a.splits)) * MID_BK;
+    const int nt = v / a.tm, m0 = (v - nt * a.tm) * 16 * MB, n0 = nt * 16 * NB * NW;
+    const int nk = a.K / MID_BK;
 
     if (wave >= NW) {
         // Direct load i of loader wave lw fills rows 8d..8d+7 of the stage, d =
         // lw + LW i: lane l the chunk position l % 8 of row 8d + l / 8.  Rows
         // past M re-read the last row: in bounds, results not stored.
         const int lw = wave - NW;
-        const bf16_t* xb = a.x + (int64_t)m0 * a.ldx + kb;
+        const bf16_t* xb = a.x + (int64_t)m0 * a.ldx;
         uint32_t voff[PER];
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
@@ -179,7 +171,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     // row 16i + 8h + n % 8; else the operand itself, chunk 4h + g of row
     // 16i + n.  Rows past N re-read the last row.
     constexpr int RING = mid_ring(MB, NB, NW, NT);
-    const char* wb = reinterpret_cast<const char*>(a.w + (int64_t)row0 * a.K + kb);
+    const char* wb = reinterpret_cast<const char*>(a.w + (int64_t)row0 * a.K);
     int woff[NB][2];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -283,9 +275,7 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
         for (int i = 0; i < NB; ++i) {
             const int col = row0 + 16 * i + 4 * g;
             if (col >= a.N) continue;
-            if (a.epi == EPI_PARTIAL)
-                *reinterpret_cast<f32x4_t*>(a.part + ((int64_t)split * a.M + m) * a.N + col) = acc[i][j];
-            else if (a.epi == Q3_EPI_SWIGLU)
+            if (a.epi == Q3_EPI_SWIGLU)
                 store4<Q3_EPI_SWIGLU>(a.y, a.ldy, m, col, acc[i][j]);
             else if (a.epi == Q3_EPI_RESID)
                 store4<Q3_EPI_RESID>(a.y, a.ldy, m, col, acc[i][j]);
@@ -295,10 +285,9 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     }
 }
 
-// Launch shape: MB token blocks x NB NW weight blocks of 16 per workgroup, and
-// the K splits.
+// Launch shape: MB token blocks x NB NW weight blocks of 16 per workgroup.
 struct MidPlan {
-    int mb, nb, nw, splits;
+    int mb, nb, nw;
 };
 
 // The tile shapes that are built, as NB, NW.
@@ -309,18 +298,18 @@ constexpr int MID_MAX_MB = 8;
 // arithmetic, so a step costs about 20 ns per 16-row block that the workgroup
 // loads (weights or tokens) plus 100 ns of barrier and latency, once per round
 // of workgroups over the CUs.
-inline MidPlan mid_plan(int M, int N, int cus, int splits = 1) {
+inline MidPlan mid_plan(int M, int N, int cus) {
     const int mblocks = (M + 15) / 16, nblocks = (N + 15) / 16;
-    MidPlan best{1, 1, 2, splits};
+    MidPlan best{1, 1, 2};
     double best_cost = 1e30;
     for (const auto& sh : MID_SHAPES) {
         const int wb = sh[0] * sh[1];
         for (int mb = mblocks < MID_MAX_MB ? mblocks : MID_MAX_MB; mb >= 1; --mb) {
             const int64_t tiles = (int64_t)((mblocks + mb - 1) / mb) * ((nblocks + wb - 1) / wb);
-            const double cost = (5 + wb + mb) * (double)((tiles * splits + cus - 1) / cus);
+            const double cost = (5 + wb + mb) * (double)((tiles + cus - 1) / cus);
             if (cost < best_cost) {
                 best_cost = cost;
-                best = {mb, sh[0], sh[1], splits};
+                best = {mb, sh[0], sh[1]};
             }
         }
     }
@@ -328,8 +317,7 @@ inline MidPlan mid_plan(int M, int N, int cus, int splits = 1) {
 }
 
 template <int MB>
-int launch_mid_mb(const MidPlan& p, const MidArgs& a, hipStream_t stream) {
-    const dim3 grid((unsigned)(a.tm * a.tn * a.splits));
+int launch_mid_mb(const MidPlan& p, const MidArgs& a, dim3 grid, hipStream_t stream) {
     switch (p.nb * 10 + p.nw) {
 #define Q3_MID(nb, nw)                                                                                           \
     case nb * 10 + nw:                                                                                           \
@@ -344,29 +332,25 @@ int launch_mid_mb(const MidPlan& p, const MidArgs& a, hipStream_t stream) {
     return (int)hipErrorInvalidValue;
 }
 
-// y = epi(x . W^T) under plan p, or with EPI_PARTIAL its K-split partials to
-// part [p.splits, M, N].
+// y = epi(x . W^T) under plan p.
 inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi,
-                      bf16_t* y, int ldy, float* part, hipStream_t stream) {
-    const bool partial = epi == EPI_PARTIAL;
-    if (!partial && epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU)
-        return (int)hipErrorInvalidValue;
-    if (partial != (part != nullptr) || (p.splits > 1 && !partial)) return (int)hipErrorInvalidValue;
+                      bf16_t* y, int ldy, hipStream_t stream) {
+    if (epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU) return (int)hipErrorInvalidValue;
     const int tm = (M + 16 * p.mb - 1) / (16 * p.mb), tn = (N + 16 * p.nb * p.nw - 1) / (16 * p.nb * p.nw);
-    if ((int64_t)tm * tn * p.splits > (1 << 30)) return (int)hipErrorInvalidValue;
-    const MidArgs a{x, ldx, w, M, N, K, epi, y, ldy, part, tm, tn, p.splits};
-    int rc = (int)hipErrorInvalidValue;
+    if ((int64_t)tm * tn > (1 << 30)) return (int)hipErrorInvalidValue;
+    const MidArgs a{x, ldx, w, M, N, K, epi, y, ldy, tm};
+    const dim3 grid((unsigned)(tm * tn));
     switch (p.mb) {
-        case 1: rc = launch_mid_mb<1>(p, a, stream); break;
-        case 2: rc = launch_mid_mb<2>(p, a, stream); break;
-        case 3: rc = launch_mid_mb<3>(p, a, stream); break;
-        case 4: rc = launch_mid_mb<4>(p, a, stream); break;
-        case 5: rc = launch_mid_mb<5>(p, a, stream); break;
-        case 6: rc = launch_mid_mb<6>(p, a, stream); break;
-        case 7: rc = launch_mid_mb<7>(p, a, stream); break;
-        case 8: rc = launch_mid_mb<8>(p, a, stream); break;
+        case 1: return launch_mid_mb<1>(p, a, grid, stream);
+        case 2: return launch_mid_mb<2>(p, a, grid, stream);
+        case 3: return launch_mid_mb<3>(p, a, grid, stream);
+        case 4: return launch_mid_mb<4>(p, a, grid, stream);
+        case 5: return launch_mid_mb<5>(p, a, grid, stream);
+        case 6: return launch_mid_mb<6>(p, a, grid, stream);
+        case 7: return launch_mid_mb<7>(p, a, grid, stream);
+        case 8: return launch_mid_mb<8>(p, a, grid, stream);
     }
-    return rc;
+    return (int)hipErrorInvalidValue;
 }
 
 }  // namespace q3gemm

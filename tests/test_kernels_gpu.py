@@ -558,7 +558,7 @@ def test_gemm_partials(M, N, K):
 @pytest.mark.parametrize("M,N,K,splits", [(1, 36, 192, 3), (17, 260, 704, 2), (45, 2560, 9728, 8), (100, 2560, 4096, 16),
                                           (129, 1028, 832, 5), (255, 2560, 9728, 1)])
 def test_gemm_partials_short_prompt(M, N, K, splits):
-    """q3_gemm_partials below 256 tokens, on the short-prompt tiling: ragged token and weight tiles, uneven K ranges
+    """q3_gemm_partials below 256 tokens, where its one token tile is ragged: ragged weight tiles, uneven K ranges
     and one step per split; the partials summed in split order against float64 on sampled rows, nothing written past
     splits * M * N floats."""
     x, w = rnd((M, K), 1.0, M + 71), rnd((N, K), 0.02, N + K + 71)
