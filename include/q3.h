@@ -79,7 +79,8 @@ int q3_gemv_partials(int M, int N, int epi);
  * above 64 (engine.py:439,450,803).  With q3_gemm_tiles_wide(M, N) the
  * 256 x 256-tile kernel (eight waves, direct global-to-LDS loads) runs, else
  * one that streams the weights into MFMA operands beside loader waves for the
- * tokens (tiles of 16..128 tokens x 32..256 weight rows).  K % 64 == 0; N % 4 == 0; ldx >= K, ldx % 8 == 0;
+ * tokens (tiles of 16..128 tokens x 32..256 weight rows), or for short K and
+ * many weight rows 16..128-row tiles.  K % 64 == 0; N % 4 == 0; ldx >= K, ldx % 8 == 0;
  * ldy % 4 == 0 (SWIGLU writes N/2 columns); x, W 16-byte and y 8-byte
  * aligned. */
 int q3_gemm(const uint16_t *x, int ldx, const uint16_t *w, int M, int N, int K,

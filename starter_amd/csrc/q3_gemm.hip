@@ -6,7 +6,7 @@
 // same epilogues as the decode GEMV (residual join, SwiGLU on interleaved
 // gate/up rows), so the prompt pass needs no separate row kernels.
 //
-// Two tilings, picked by the number of output tiles:
+// Three tilings, picked by the number of output tiles and the K steps:
 //
 // * wide (the prompt pass): a 512-thread workgroup owns a 256 x 256 output
 //   tile; eight waves, two per SIMD, each a 128 (token) x 64 (weight row)
@@ -37,7 +37,10 @@
 //
 // * mid (few tiles: short prompts and decode batches above 64): weights
 //   straight into MFMA operands, token rows through LDS by loader waves
-//   (q3_gemm_mid.hpp).
+//   (q3_gemm_mid.hpp);
+//
+// * narrow (few tiles, and few K steps or several rounds of the mid tiles): 256
+//   threads, BM x BN tiles of up to 128 x 128, LDS staged through registers.
 //
 // Operands: A = W rows (n), B = x rows (m), so a lane's four C values are four
 // consecutive output columns of one token row (both halves of a SwiGLU pair in
@@ -335,6 +338,143 @@ __global__ __launch_bounds__(256) void wide_tail_reduce_kernel(const float* __re
     store4<EPI>(y, ldy, m0 + r, n0 + c, a);
 }
 
+// ---------------------------------------------------------------- narrow
+
+constexpr int NARROW_THREADS = 256;
+constexpr int NARROW_BK = 64;
+
+template <int BM, int BN, int WM, int WN, int EPI>
+__global__ __launch_bounds__(NARROW_THREADS) void gemm_narrow_kernel(const bf16_t* __restrict__ x, int ldx,
+                                                       const bf16_t* __restrict__ w, int M, int N, int K,
+                                                       bf16_t* y, int ldy) {
+    constexpr int TM = BM / WM, TN = BN / WN;
+    constexpr int FM = TM / 16, FN = TN / 16;
+    constexpr int XCH = BM * 8, WCH = BN * 8;  // 16-byte chunks per tile
+    constexpr int XPT = (XCH + NARROW_THREADS - 1) / NARROW_THREADS, WPT = (WCH + NARROW_THREADS - 1) / NARROW_THREADS;
+    static_assert(WM * WN == 4, "4 waves");
+
+    __shared__ __align__(16) bf16_t xs[BM * NARROW_BK];
+    __shared__ __align__(16) bf16_t ws[BN * NARROW_BK];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int g = lane >> 4, n = lane & 15;
+    const int wm = wave / WN, wn = wave % WN;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+
+    uint4 xr[XPT], wr[WPT];
+    auto gload = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < XPT; ++j) {
+            const int e = tid + j * NARROW_THREADS;
+            const int r = e >> 3, c = e & 7;
+            xr[j] = make_uint4(0, 0, 0, 0);
+            if (e < XCH && m0 + r < M)
+                xr[j] = *reinterpret_cast<const uint4*>(x + (int64_t)(m0 + r) * ldx + k0 + 8 * c);
+        }
+#pragma unroll
+        for (int j = 0; j < WPT; ++j) {
+            const int e = tid + j * NARROW_THREADS;
+            const int r = e >> 3, c = e & 7;
+            wr[j] = make_uint4(0, 0, 0, 0);
+            if (e < WCH && n0 + r < N)
+                wr[j] = load_nt((w + (int64_t)(n0 + r) * K + k0 + 8 * c));
+        }
+    };
+    auto sstore = [&]() {
+#pragma unroll
+        for (int j = 0; j < XPT; ++j) {
+            const int e = tid + j * NARROW_THREADS;
+            if (e < XCH) {
+                const int r = e >> 3, c = e & 7;
+                *reinterpret_cast<uint4*>(xs + r * NARROW_BK + (c ^ wide_swz(r)) * 8) = xr[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < WPT; ++j) {
+            const int e = tid + j * NARROW_THREADS;
+            if (e < WCH) {
+                const int r = e >> 3, c = e & 7;
+                *reinterpret_cast<uint4*>(ws + r * NARROW_BK + (c ^ wide_swz(r)) * 8) = wr[j];
+            }
+        }
+    };
+
+    f32x4_t acc[FN][FM];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    gload(0);
+    for (int k0 = 0; k0 < K; k0 += NARROW_BK) {
+        __syncthreads();
+        sstore();
+        __syncthreads();
+        if (k0 + NARROW_BK < K) gload(k0 + NARROW_BK);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            u32x4_t av[FN], bv[FM];
+#pragma unroll
+            for (int i = 0; i < FN; ++i) {
+                const int r = wn * TN + 16 * i + n;
+                av[i] = *reinterpret_cast<const u32x4_t*>(ws + r * NARROW_BK + ((4 * kk + g) ^ wide_swz(r)) * 8);
+            }
+#pragma unroll
+            for (int j = 0; j < FM; ++j) {
+                const int r = wm * TM + 16 * j + n;
+                bv[j] = *reinterpret_cast<const u32x4_t*>(xs + r * NARROW_BK + ((4 * kk + g) ^ wide_swz(r)) * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < FN; ++i)
+#pragma unroll
+                for (int j = 0; j < FM; ++j) acc[i][j] = mfma(av[i], bv[j], acc[i][j]);
+        }
+    }
+
+    // acc[i][j][e] = C[token m0 + TM*wm + 16j + n][column n0 + TN*wn + 16i + 4g + e].
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+        const int m = m0 + wm * TM + 16 * j + n;
+        if (m >= M) continue;
+#pragma unroll
+        for (int i = 0; i < FN; ++i) {
+            const int col = n0 + wn * TN + 16 * i + 4 * g;
+            if (col < N) store4<EPI>(y, ldy, m, col, acc[i][j]);
+        }
+    }
+}
+
+template <int BM, int BN, int WM, int WN>
+int launch_narrow_tile(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y, int ldy,
+           hipStream_t stream) {
+    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    switch (epi) {
+        case Q3_EPI_STORE:
+            Q3_LAUNCH((gemm_narrow_kernel<BM, BN, WM, WN, Q3_EPI_STORE>), grid, dim3(NARROW_THREADS), 0, stream, x, ldx, w, M, N,
+                      K, y, ldy);
+            break;
+        case Q3_EPI_RESID:
+            Q3_LAUNCH((gemm_narrow_kernel<BM, BN, WM, WN, Q3_EPI_RESID>), grid, dim3(NARROW_THREADS), 0, stream, x, ldx, w, M, N,
+                      K, y, ldy);
+            break;
+        case Q3_EPI_SWIGLU:
+            Q3_LAUNCH((gemm_narrow_kernel<BM, BN, WM, WN, Q3_EPI_SWIGLU>), grid, dim3(NARROW_THREADS), 0, stream, x, ldx, w, M, N,
+                      K, y, ldy);
+            break;
+        default:
+            return (int)hipErrorInvalidValue;
+    }
+    Q3_CHECK_LAUNCH();
+}
+
+int launch_narrow(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi, bf16_t* y, int ldy,
+                  hipStream_t stream) {
+    if (M <= 16) return launch_narrow_tile<16, 64, 1, 4>(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    if (M <= 32) return launch_narrow_tile<32, 64, 2, 2>(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    if (M <= 64) return launch_narrow_tile<64, 64, 2, 2>(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    return launch_narrow_tile<128, 128, 2, 2>(x, ldx, w, M, N, K, epi, y, ldy, stream);
+}
+
 // Whole tiles 0..full-1, then the rest split `splits` ways (EPI_PARTIAL:
 // full == 0, partials [splits, M, N]; other epilogues: compact partials
 // finished by wide_tail_reduce_kernel, launched here after the GEMM).
@@ -404,6 +544,35 @@ static int mid_cus() {
     return cus > 0 ? cus : 256;
 }
 
+// Where the narrow tiles beat the mid plan p (us below: narrow / mid).  The
+// lines are drawn through 2981 shapes of 1-4095 tokens, 4-262144 weight rows
+// and K of 64-10240; seven of them are more than 5% slower than the narrow
+// tiles would be (9% at most), 39 more than 10% slower than the faster of the
+// two.
+//  * One or two K steps: the mid pipeline's prologue is not repaid (64 x 64 x
+//    64 at 16 tokens 2.1 / 2.7); nor with its large tiles up to nine steps (300
+//    tokens, 16384 rows, K = 64 / 320: 6.9 / 9.0, 11.3 / 13.0).
+//  * More weight rows than a round of 160-row workgroups takes, and the rounds
+//    of the larger ones a quarter empty (129 tokens, 45272 rows of 4096: 139.7
+//    / 149.2).
+//  * Several rounds, of which a CU holds one or two mid workgroups at a time,
+//    where the last one is mostly idle, K is short or one token block leaves
+//    the weight streams alone.  The narrow workgroups are shorter and three
+//    share a CU (the LM head, 151936 rows of 2560, at 9 / 16 / 100 / 128 tokens
+//    132 / 135 / 183 / 192 against 146 / 149 / 197 / 209).  Not at 49-64 tokens,
+//    whose narrow tiles are 64 x 64 and read the tokens twice as often (LM head
+//    at 64: 188 / 178), nor above 128, where narrow takes two token tiles (344 /
+//    272 at 129).
+static bool narrow_faster(const MidPlan& p, int M, int N, int K, int cus) {
+    const int steps = K / MID_BK, blocks = p.mb + p.nb * p.nw;
+    if (steps <= 2 && (M <= 64 || blocks >= 15)) return true;
+    if (steps <= 9 && blocks >= 16) return true;
+    const int64_t tiles = mid_tiles(p, M, N), slots = (tiles + cus - 1) / cus * cus;
+    if (N > 160 * cus && 4 * tiles < 3 * slots) return true;
+    return M <= 128 && tiles > cus &&
+           (M <= 16 || steps <= 16 || ((M <= 48 || M > 64) && 10 * tiles < 9 * slots));
+}
+
 extern "C" int q3_gemm_tiles_wide(int M, int N) {
     if (M < 256 || N < 1) return 0;
     const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -421,7 +590,9 @@ extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, 
     if (q3_gemm_tiles_wide(M, N))
         return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, ((M + 255) / 256) * ((N + 255) / 256), 1, nullptr,
                            stream);
-    return launch_mid(mid_plan(M, N, mid_cus()), x, ldx, w, M, N, K, epi, y, ldy, stream);
+    const MidPlan plan = mid_plan(M, N, mid_cus());
+    if (narrow_faster(plan, M, N, K, mid_cus())) return launch_narrow(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    return launch_mid(plan, x, ldx, w, M, N, K, epi, y, ldy, stream);
 }
 
 // Split tail of the wide tiling.  One 256 x 256-tile workgroup fits a CU

@@ -290,6 +290,10 @@ struct MidPlan {
     int mb, nb, nw;
 };
 
+inline int64_t mid_tiles(const MidPlan& p, int M, int N) {
+    return (int64_t)((M + 16 * p.mb - 1) / (16 * p.mb)) * ((N + 16 * p.nb * p.nw - 1) / (16 * p.nb * p.nw));
+}
+
 // The tile shapes that are built, as NB, NW.
 constexpr int MID_SHAPES[][2] = {{1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 3}, {2, 5}, {2, 8}};
 constexpr int MID_MAX_MB = 8;
@@ -336,10 +340,10 @@ int launch_mid_mb(const MidPlan& p, const MidArgs& a, dim3 grid, hipStream_t str
 inline int launch_mid(const MidPlan& p, const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, int epi,
                       bf16_t* y, int ldy, hipStream_t stream) {
     if (epi != Q3_EPI_STORE && epi != Q3_EPI_RESID && epi != Q3_EPI_SWIGLU) return (int)hipErrorInvalidValue;
-    const int tm = (M + 16 * p.mb - 1) / (16 * p.mb), tn = (N + 16 * p.nb * p.nw - 1) / (16 * p.nb * p.nw);
-    if ((int64_t)tm * tn > (1 << 30)) return (int)hipErrorInvalidValue;
-    const MidArgs a{x, ldx, w, M, N, K, epi, y, ldy, tm};
-    const dim3 grid((unsigned)(tm * tn));
+    const int64_t tiles = mid_tiles(p, M, N);
+    if (tiles > (1 << 30)) return (int)hipErrorInvalidValue;
+    const MidArgs a{x, ldx, w, M, N, K, epi, y, ldy, (M + 16 * p.mb - 1) / (16 * p.mb)};
+    const dim3 grid((unsigned)tiles);
     switch (p.mb) {
         case 1: return launch_mid_mb<1>(p, a, grid, stream);
         case 2: return launch_mid_mb<2>(p, a, grid, stream);

@@ -431,6 +431,38 @@ def test_gemm_short_prompt_tiles(M, N, K):
         assert torch.all(ws.cpu() == 9.0)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (16, 68, 64), (17, 1028, 128), (33, 260, 64), (64, 132, 128),
+                                   (300, 16388, 64), (129, 16384, 320), (1, 98308, 320), (9, 151936, 320),
+                                   (16, 98308, 1088), (33, 98308, 320), (100, 98308, 1088), (128, 151936, 320),
+                                   (161, 45272, 640)])
+def test_gemm_narrow_tiles(M, N, K):
+    """Shapes of few K steps, or of weights that take the short-prompt tiles several rounds, run on the narrow tiles:
+    ragged ones against float64, and bit for bit what the other tilings give for the same sums (at most 2048 of the
+    weight rows, or 65 tokens, at a time take those)."""
+    rows = max(M, 65)
+    x, w = rnd((rows, K), 1.0, M + 81), rnd((N, K), 0.02, N + K + 81)
+    xd, wd = dv(x), dv(w)
+
+    def run(m, lo, n, epi, fill):  # weight rows lo..lo + n - 1 over the columns of fill
+        cols = fill.shape[1]
+        out = torch.full((rows, (cols + 7) // 4 * 4), 5.0, dtype=torch.bfloat16)
+        out[:, :cols] = fill
+        out = dv(out)
+        call("q3_gemm", P(xd), K, P(wd) + 2 * lo * K, m, n, K, epi, P(out), out.shape[1], S())
+        torch.cuda.synchronize()
+        out = out.cpu()
+        assert torch.all(out[:, cols:] == 5.0) and torch.equal(out[m:, :cols], fill[m:])
+        return out[:m, :cols].contiguous()
+
+    for epi, per in ((_lib.EPI_STORE, 1), (_lib.EPI_RESID, 1), (_lib.EPI_SWIGLU, 2)):
+        fill = rnd((rows, N // per), 1.0, 82)
+        y = run(M, 0, N, epi, fill)
+        parts = [run(rows, lo, min(2048, N - lo), epi, fill[:, lo // per:(lo + 2048) // per]) for lo in range(0, N, 2048)]
+        assert torch.equal(y, torch.cat(parts, 1)[:M]), epi
+        if epi == _lib.EPI_STORE:
+            check_projection(y[:, -2000:], x[:M], w[-2000:], frac=0.03 if N > 100 else 0.5)
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(4096, 6144, 2560, _lib.EPI_STORE), (4096, 2560, 4096, _lib.EPI_RESID),
                                        (2600, 19456, 2560, _lib.EPI_SWIGLU), (4096, 2560, 9728, _lib.EPI_RESID),
                                        (3000, 3800, 320, _lib.EPI_STORE), (40961, 4096, 64, _lib.EPI_STORE)])
