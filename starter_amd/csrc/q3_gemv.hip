@@ -162,6 +162,12 @@ constexpr int stage_rows = XMODE == Q3_X_NORM ? (M + norm_groups(W) - 1) / norm_
 template <int XMODE, int W>
 constexpr int stage_threads = XMODE == Q3_X_NORM ? GEMV_THREADS : W * Q3_WAVE;
 
+// The group of this thread (a constant where there is one).
+template <int XMODE, int W>
+__device__ __forceinline__ int stage_group() {
+    return XMODE == Q3_X_NORM && norm_groups(W) > 1 ? (int)threadIdx.x / stage_threads<XMODE, W> : 0;
+}
+
 template <int XMODE, int KU, int W>
 constexpr int x_chunks() {
     return (64 * KU + stage_threads<XMODE, W> - 1) / stage_threads<XMODE, W>;
@@ -172,7 +178,7 @@ __device__ __forceinline__ void stage_x_issue(const GemvArgs& a,
                                               u32x4_t (&xv)[x_chunks<XMODE, KU, W>()][stage_rows<M, XMODE, W>],
                                               u32x4_t (&gv)[x_chunks<XMODE, KU, W>()]) {
     constexpr int XC = x_chunks<XMODE, KU, W>(), MG = stage_rows<M, XMODE, W>, NT = stage_threads<XMODE, W>;
-    const int tid = threadIdx.x % NT, m0 = threadIdx.x / NT * MG;
+    const int grp = stage_group<XMODE, W>(), tid = threadIdx.x - grp * NT, m0 = grp * MG;
 #pragma unroll
     for (int j = 0; j < XC; ++j) {
         const int c = min(tid + j * NT, 64 * KU - 1);  // past the row: a duplicate, never used
@@ -189,7 +195,7 @@ __device__ __forceinline__ void stage_x_finish(const GemvArgs& a,
                                                const u32x4_t (&gv)[x_chunks<XMODE, KU, W>()], bf16_t* xs) {
     constexpr int XC = x_chunks<XMODE, KU, W>(), MG = stage_rows<M, XMODE, W>, NT = stage_threads<XMODE, W>;
     constexpr int K = 512 * KU;
-    const int tid = threadIdx.x % NT, grp = threadIdx.x / NT, m0 = grp * MG;
+    const int grp = stage_group<XMODE, W>(), tid = threadIdx.x - grp * NT, m0 = grp * MG;
     if constexpr (XMODE == Q3_X_PLAIN) {
 #pragma unroll
         for (int j = 0; j < XC; ++j) {
