@@ -445,17 +445,19 @@ constexpr bool combo_used(int xmode, int epi) {
 // Waves per workgroup.  A CU streams at most ~27 GB/s, so a launch is as slow
 // as its most loaded CU: plain-input projections take five waves when that
 // spreads the rows more evenly over the 256 CUs (N = 2560: 512 workgroups,
-// two per CU, against 640 = 2.5 per CU with four).  From three batch rows on
-// ten waves do the same with one staging of the rows per CU instead of two
-// (K = 9728: they are 58 KB at three rows, 78 at four; 12.0 / 15.0 -> 10.9 /
-// 12.1 us).
-int waves_for(int xmode, int epi, int M, int N) {
+// two per CU, against 640 = 2.5 per CU with four).  At three and four batch
+// rows of long K ten waves do the same with one staging of the rows per CU
+// instead of two (us, five -> ten, 2560 rows: K = 9728, where they are 58 KB at
+// three rows and 78 at four, 12.3 / 15.1 -> 11.0 / 12.2; K = 4096 6.0 / 6.5 ->
+// 5.7 / 6.5).  At K = 2560 the wider barrier costs more than the staging: 4.7 /
+// 5.0 -> 4.7 / 5.4, 7680 rows 8.7 / 9.3 -> 9.7 / 10.5.
+int waves_for(int xmode, int epi, int M, int N, int K) {
     constexpr int CUS = 256;
     if (xmode != Q3_X_PLAIN || epi == Q3_EPI_ARGMAX || epi == Q3_EPI_STORE_ARGMAX) return GEMV_WAVES;
     const int units = N / rows_per_wave(M, epi);
     auto load = [&](int w) { return ((units + w - 1) / w + CUS - 1) / CUS * w; };
     if (load(5) >= load(GEMV_WAVES)) return GEMV_WAVES;
-    return (M == 3 || M == 4) && load(10) == load(5) ? 10 : 5;
+    return (M == 3 || M == 4) && K >= 4096 && load(10) == load(5) ? 10 : 5;
 }
 
 template <int M, int KU, int XMODE, bool XLDS, int EPI, int W>
@@ -472,8 +474,8 @@ int launch_w(const GemvArgs& a, hipStream_t stream) {
 template <int M, int KU, int XMODE, bool XLDS, int EPI>
 int launch_one(const GemvArgs& a, hipStream_t stream) {
     if constexpr (XMODE == Q3_X_PLAIN && EPI != Q3_EPI_ARGMAX && EPI != Q3_EPI_STORE_ARGMAX) {
-        const int w = waves_for(XMODE, EPI, M, a.N);
-        if constexpr (KU > 0 && (M == 3 || M == 4)) {
+        const int w = waves_for(XMODE, EPI, M, a.N, a.K);
+        if constexpr (KU >= 8 && (M == 3 || M == 4)) {
             if (w == 10) return launch_w<M, KU, XMODE, true, EPI, 10>(a, stream);
         }
         if (w >= 5) return launch_w<M, KU, XMODE, XLDS, EPI, 5>(a, stream);
