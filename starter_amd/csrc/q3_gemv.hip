@@ -32,9 +32,10 @@
 
 namespace {
 
-constexpr int GEMV_THREADS = 256;  // four waves; plain-input launches may take five
+constexpr int GEMV_THREADS = 256;  // four waves; see waves_for
 constexpr int GEMV_WAVES = GEMV_THREADS / Q3_WAVE;
-constexpr int LDS_X_LIMIT = 60 * 1024;
+constexpr int LDS_X_LIMIT = 60 * 1024;  // input rows in dynamic LDS
+constexpr int LDS_X_FIXED = 80 * 1024;  // and in a static array (ten waves): two workgroups per CU
 
 struct GemvArgs {
     const bf16_t* x;      // X_PLAIN: input rows; X_NORM: rows to normalise; X_EMBED_NORM: table
@@ -344,12 +345,13 @@ __device__ void argmax_epilogue(const GemvArgs& a, const float (&acc)[R][M], int
 }
 
 // KU > 0: K == 512*KU, all weight loads issued up front.  KU == 0: any K % 8 == 0.
-// W waves per workgroup (four, or five or ten for plain inputs; ten keep the
-// input rows in a static array, which may pass 64 KB).
+// W waves per workgroup (waves_for); ten keep the input rows in a static array,
+// which may pass the 64 KB that dynamic LDS has by default.
 template <int M, int R, int KU, int XMODE, bool XLDS, int EPI, int W>
 __global__ __launch_bounds__(W * Q3_WAVE) void gemv_dot2_kernel(GemvArgs a) {
     static_assert(W == GEMV_WAVES || (EPI != Q3_EPI_ARGMAX && EPI != Q3_EPI_STORE_ARGMAX),
                   "the argmax epilogue is written for four waves");
+    static_assert(W != 10 || M * 512 * KU * 2 <= LDS_X_FIXED, "input rows of a ten-wave workgroup");
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ __align__(16) bf16_t fixed[W == 10 ? M * 512 * KU : 8];
     bf16_t* xs = W == 10 ? fixed : reinterpret_cast<bf16_t*>(smem);
@@ -442,6 +444,11 @@ constexpr bool combo_used(int xmode, int epi) {
          : true;
 }
 
+// The normed projections that are built with eight waves too.
+constexpr bool eight_waves_built(int M, int K, int epi) {
+    return epi == Q3_EPI_STORE && ((K == 2560 && M >= 2) || (K == 4096 && M >= 3 && M <= 6));
+}
+
 // Waves per workgroup.  A CU streams at most ~27 GB/s, so a launch is as slow
 // as its most loaded CU: plain-input projections take five waves when that
 // spreads the rows more evenly over the 256 CUs (N = 2560: 512 workgroups,
@@ -451,8 +458,19 @@ constexpr bool combo_used(int xmode, int epi) {
 // three rows and 78 at four, 12.3 / 15.1 -> 11.0 / 12.2; K = 4096 6.0 / 6.5 ->
 // 5.7 / 6.5).  At K = 2560 the wider barrier costs more than the staging: 4.7 /
 // 5.0 -> 4.7 / 5.4, 7680 rows 8.7 / 9.3 -> 9.7 / 10.5.
+//
+// Stored normed projections whose four-wave workgroups outnumber the CUs take
+// eight waves, which share one staging (us, four -> eight, K = 2560: 1280 rows
+// at 2 / 4 / 8 batch rows 4.6 / 6.5 / 10.6 -> 3.9 / 5.4 / 7.7, 6144 rows 8.7 /
+// 12.3 / 25.0 -> 7.9 / 10.2 / 15.8, 151936 rows 121 / 229 / 540 -> 116 / 157 /
+// 290).  With a CU or more per four-wave workgroup they would halve the CUs at
+// work (1024 rows 3.4 / 4.7 / 7.4 -> 3.8 / 5.2 / 7.6).  At K = 4096 two and
+// seven batch rows are as fast or faster with four (2560 rows 6.6 / 13.3 -> 6.9
+// / 13.9, 151936 at two 188 -> 191).  SwiGLU, four rows a wave, is slower with
+// eight (17.4 / 18.9 / 21.5 -> 19.1 / 24.0 / 26.1 at 2 / 3 / 4 batch rows).
 int waves_for(int xmode, int epi, int M, int N, int K) {
     constexpr int CUS = 256;
+    if (xmode == Q3_X_NORM && eight_waves_built(M, K, epi)) return N > GEMV_WAVES * CUS ? 2 * GEMV_WAVES : GEMV_WAVES;
     if (xmode != Q3_X_PLAIN || epi == Q3_EPI_ARGMAX || epi == Q3_EPI_STORE_ARGMAX) return GEMV_WAVES;
     const int units = N / rows_per_wave(M, epi);
     auto load = [&](int w) { return ((units + w - 1) / w + CUS - 1) / CUS * w; };
@@ -480,12 +498,9 @@ int launch_one(const GemvArgs& a, hipStream_t stream) {
         }
         if (w >= 5) return launch_w<M, KU, XMODE, XLDS, EPI, 5>(a, stream);
     }
-    // Stored normed projections of two rows on: eight waves share one staging
-    // (us, four -> eight waves, rows 2 / 3 / 4: 6144 rows 8.7 / 10.5 / 12.5 ->
-    // 7.7 / 9.0 / 10.1; 151936 rows 120 / 167 / 230 -> 110 / 135 / 155).  SwiGLU,
-    // four rows a wave, is slower so (17.4 / 18.9 / 21.5 -> 19.1 / 24.0 / 26.1).
-    if constexpr (XMODE == Q3_X_NORM && KU > 0 && M >= 2 && EPI == Q3_EPI_STORE) {
-        return launch_w<M, KU, XMODE, XLDS, EPI, 2 * GEMV_WAVES>(a, stream);
+    if constexpr (XMODE == Q3_X_NORM && KU > 0 && eight_waves_built(M, 512 * KU, EPI)) {
+        if (waves_for(XMODE, EPI, M, a.N, a.K) == 2 * GEMV_WAVES)
+            return launch_w<M, KU, XMODE, XLDS, EPI, 2 * GEMV_WAVES>(a, stream);
     }
     return launch_w<M, KU, XMODE, XLDS, EPI, GEMV_WAVES>(a, stream);
 }
@@ -555,7 +570,7 @@ extern "C" int q3_gemv(int x_mode, const bf16_t* x, int ldx, const int64_t* ids,
                        int epi, bf16_t* y, int ldy, float* part_val, int* part_idx,
                        const int64_t* pos, const int64_t* feed, int* rec, int npos, hipStream_t stream) {
     if (M < 1 || M > Q3_GEMV_MAX_M || N < 1 || K < 8 || (K % 8) != 0) return (int)hipErrorInvalidValue;
-    // Staged rows live in LDS (M*K BF16, within the 64 KiB default).
+    // Normalised rows are staged in dynamic LDS (M*K BF16, within its 64 KiB default).
     if (x_mode != Q3_X_PLAIN && (K > Q3_GEMV_MAX_NORM_K || (size_t)M * K * 2 > LDS_X_LIMIT))
         return (int)hipErrorInvalidValue;
     if (epi == Q3_EPI_SWIGLU && (N % 2) != 0) return (int)hipErrorInvalidValue;

@@ -182,11 +182,11 @@ def test_gemv_plain_store(M, N, K):
     check_projection(y, x, w)
 
 
-@pytest.mark.parametrize("M", [2, 3, 4, 5])
-@pytest.mark.parametrize("N,K", [(1, 2560), (333, 2560), (6151, 2560), (2555, 9728), (2557, 4096)])
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 7])
+@pytest.mark.parametrize("N,K", [(1, 2560), (333, 2560), (6151, 2560), (2555, 9728), (2557, 4096), (1024, 2560), (1025, 4096)])
 def test_gemv_large_workgroups(M, N, K):
-    """Ten-wave workgroups (plain input, three and four rows, the 2560-wide long-K shapes) and eight-wave ones (X_NORM,
-    two groups of four waves staging half the rows each), with waves past the last row: the plain projection against
+    """Ten-wave workgroups (plain input, three and four rows, the 2560-wide long-K shapes) and eight-wave ones (X_NORM
+    past 1024 weight rows, two groups of four waves staging half the rows each), with waves past the last row: the plain projection against
     float64, the residual join and the normed projection bit for bit against it, nothing written past N columns."""
     x, w, res = rnd((M, K), 1.0, M), rnd((N, K), 0.02, N + K), rnd((M, N + 8), 1.0, 7)
     xd, wd, g = dv(x), dv(w), dv((1 + rnd((K,), 0.2, 8).float()).to(torch.bfloat16))
