@@ -111,7 +111,7 @@ def test_prompt_gemm_split_policy():
     assert _lib.call("q3_gemm_splits", 512, H, 4096) == 12
     assert _lib.call("q3_gemm_splits", 3840, H, 4096) == 3
     assert _lib.call("q3_gemm_splits", 3072, H, 9728) == 2
-    assert _lib.call("q3_gemm_splits", 255, H, 4096) == 0       # narrow tiles
+    assert _lib.call("q3_gemm_splits", 255, H, 4096) == 0       # short-prompt tiles
     assert _lib.call("q3_gemm_splits", 4096, H, 4096) == 0      # 160 whole tiles
     assert _lib.call("q3_gemm_splits", 8192, H, 9728) == 0
     assert _lib.call("q3_gemm_splits", 1024, H, 320) == 0       # 5 K steps: no split of >= 4 steps

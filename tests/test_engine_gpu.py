@@ -113,7 +113,7 @@ def test_yield_contract(tiny_engine):
         list(tiny_engine.generate([[1, 2, 512]], 2))  # id outside the vocabulary
 
 
-@pytest.mark.parametrize("batch", [9, 12])
+@pytest.mark.parametrize("batch", [9, 12, 100])
 def test_large_batch_path_matches_oracle(tiny_engine, tiny_ckpt, batch):
     """B > 8 takes the MFMA GEMM path; rows are checked against the CPU oracle."""
     cfg, tensors = load_checkpoint(tiny_ckpt)

@@ -431,6 +431,45 @@ def test_gemm_short_prompt_tiles(M, N, K):
         assert torch.all(ws.cpu() == 9.0)
 
 
+# One ragged token count for each tile shape (token blocks, weight blocks, waves; whole-line loads with one token tile)
+# that the short-prompt planner picks on 256 CUs for the model's projections and for LM heads.
+SHORT_PROMPT_TILES = {6144: (9, 19, 45, 61, 83, 100, 147, 180, 211, 235, 247, 1300, 1470),
+                      2560: (29, 81, 100, 150, 200, 245),
+                      19456: (9, 29, 45, 61, 75, 83, 100, 121, 150, 180, 211, 235, 270, 300, 350, 400, 460),
+                      32768: (9, 29, 45, 61, 75, 90, 100, 121, 130, 170, 200, 235),
+                      50000: (61,)}
+
+
+@pytest.mark.parametrize("M,N", [(M, N) for N, tokens in SHORT_PROMPT_TILES.items() for M in tokens])
+def test_gemm_every_short_prompt_tile(M, N, K=704):
+    """Each instance of the loader-wave tiling that the model's sizes run (11 K steps: remainders of rings of three, four
+    and eight register sets): every output bit for bit the BF16 rounding of the 256 x 256 tiling's FP32 sums, sampled
+    rows against float64, the residual join and SwiGLU exactly those of the stored projection, nothing written past N or
+    M."""
+    assert call("q3_gemm_tiles_wide", M, N) == 0
+    x, w = rnd((M, K), 1.0, M + 91), rnd((N, K), 0.02, N + K + 91)
+    xd, wd, res = dv(x), dv(w), dv(rnd((M, N), 1.0, 92))
+    sums = torch.empty(M, N, device=DEV)
+    call("q3_gemm_partials", P(xd), K, P(wd), M, N, K, P(sums), 1, S())
+
+    def run(epi, fill):
+        out = torch.full((M + 2, fill.shape[1] + 4), 5.0, dtype=torch.bfloat16, device=DEV)
+        out[:M, :-4] = fill
+        call("q3_gemm", P(xd), K, P(wd), M, N, K, epi, P(out), out.shape[1], S())
+        torch.cuda.synchronize()
+        assert torch.all(out[:, -4:] == 5.0) and torch.all(out[M:] == 5.0)
+        return out[:M, :-4].contiguous()
+
+    y = run(_lib.EPI_STORE, torch.zeros_like(res))
+    assert torch.equal(y, sums.bfloat16())
+    rows = torch.tensor([0, M // 2, M - 1])
+    check_projection(y.cpu()[rows], x[rows], w)
+    assert torch.equal(run(_lib.EPI_RESID, res), (res.float() + y.float()).bfloat16())
+    act = torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV)
+    call("q3_swiglu_rows", P(y), P(act), M, N // 2, S())
+    assert torch.equal(run(_lib.EPI_SWIGLU, torch.zeros_like(act)), act)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 4, 64), (16, 68, 64), (17, 1028, 128), (33, 260, 64), (64, 132, 128),
                                    (300, 16388, 64), (129, 16384, 320), (1, 98308, 320), (9, 151936, 320),
                                    (16, 98308, 1088), (33, 98308, 320), (100, 98308, 1088), (128, 151936, 320),
@@ -491,7 +530,7 @@ def test_gemm_wide(M, N, K, epi):
         return
     # The fused epilogues against the unfused ones on the same rows: the plain
     # projection of those rows (checked above for its own bar) is recomputed
-    # here through the narrow tiling, whose sums the wide path must match to
+    # here through the short-prompt tiling, whose sums the wide path must match to
     # the same float64 bar.
     y = torch.empty(len(rows), N, dtype=torch.bfloat16, device=DEV)
     call("q3_gemm", P(dv(xs.contiguous())), K, P(wd), len(rows), N, K, _lib.EPI_STORE, P(y), N, S())

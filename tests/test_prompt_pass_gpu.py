@@ -123,7 +123,7 @@ def test_gemm_ws_full_prompt(name, N, K, epi):
     if epi == _lib.EPI_STORE:
         check_projection(got, xs, wc)
         return
-    # The plain projection of the sampled rows through the narrow tiling,
+    # The plain projection of the sampled rows through the short-prompt tiling,
     # checked against float64, then the fused epilogue against it.
     y = torch.empty(len(rows), N, dtype=torch.bfloat16, device=DEV)
     call("q3_gemm", P(xs.to(DEV)), K, P(w), len(rows), N, K, _lib.EPI_STORE, P(y), N, S())
