@@ -534,9 +534,9 @@ static int cu_count() {
 }
 
 // The wide tiling once it has at least this many 256 x 256 tiles (with fewer,
-// too many CUs would idle: o unsplit at 1000 tokens, 40 tiles, takes 34 us on
-// the mid tiling) and at least one full token tile (a 64-row LM head would
-// waste three quarters of each tile's MFMA work).
+// too many CUs would idle: q|k|v at 1536 / 2000 tokens, 144 / 192 tiles, takes
+// 80.5 us on the mid tiling / 62.0 on this one) and at least one full token tile
+// (a 64-row LM head would waste three quarters of each tile's MFMA work).
 constexpr int WIDE_MIN_TILES = 160;
 
 static int mid_cus() {
@@ -596,14 +596,18 @@ extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, 
 }
 
 // Split tail of the wide tiling.  One 256 x 256-tile workgroup fits a CU
-// (128 KB of LDS), so the tiles run in rounds of `cus`; when the last round
+// (160 KB of LDS), so the tiles run in rounds of `cus`; when the last round
 // is at most half full, its tiles are split along K over about `cus`
 // workgroups (at most TAIL_MAX_SPLITS splits of >= WIDE_SPLIT_STEPS K
 // steps), which shortens that round by the split count, and
 // wide_tail_reduce_kernel finishes them.  Below WIDE_MIN_TILES the same
 // applies to all the tiles when they fill at most half the CUs, from 256
-// tokens (qkv at 512 / 1000 tokens 38.7 / 51.0 us; whole on the mid tiling 30.3
-// / 53.6).  The partials take tail * splits <= cus tiles of 256 x 256 FP32.
+// tokens (us, split here / whole on the mid tiling: q|k|v at 256 / 512 / 768 /
+// 1000 / 1280 tokens 32.3 / 23.9, 38.1 / 31.2, 43.3 / 42.0, 50.3 / 54.8, 54.1 /
+// 57.3; gate/up at 256 52.2 / 50.0).  The mid tiling is the faster one up to
+// about 800 tokens; the split stays because the whole sums have another order,
+// and with it the prompt's near-tied tokens would change.  The partials take
+// tail * splits <= cus tiles of 256 x 256 FP32.
 struct WidePlan {
     int full, tail, splits;
 };
@@ -645,15 +649,17 @@ extern "C" int q3_gemm_ws(const bf16_t* x, int ldx, const bf16_t* w, int M, int 
 }
 
 // Split-K for the wide tiling where it has fewer than WIDE_MIN_TILES tiles:
-// at most WIDE_SPLIT_WGS workgroups (one per CU: each holds 128 KB of LDS),
+// at most WIDE_SPLIT_WGS workgroups (one per CU: each holds 160 KB of LDS),
 // or three splits from 128 tiles on, at most 16 splits (the partial
 // consumers' limit) of at least WIDE_SPLIT_STEPS K steps each; 0 where the
-// unsplit kernels apply.  Measured on MI355X (o and down of the prompt pass,
-// N = 2560, the split GEMM plus add_rmsnorm_partials against the unsplit GEMM
-// plus rmsnorm): the pick is the fastest split count at 256-3840 tokens but
-// one (512 tokens: 12 splits 34.2 us, 8 splits 32.5), and at 1024 tokens o
-// takes 41.7 against 81.3 us, down 64.3 against 175.6; at 150 tiles three
-// splits (450 workgroups) beat two and one (o: 113 / 123 / 137 us).
+// unsplit kernels apply.  Measured on MI355X (us, N = 2560: the split GEMM plus
+// add_rmsnorm_partials / the mid tiling whole plus rmsnorm): down at 256 / 512 /
+// 1000 / 2000 / 3000 tokens 38.3 / 50.6, 45.0 / 65.1, 62.4 / 88.3, 97.9 / 131.7,
+// 133.5 / 183.2; o 29.8 / 24.5, 35.2 / 31.0, 42.0 / 41.2, 57.7 / 62.3, 73.7 /
+// 86.4.  Below about 1000 tokens o would be faster whole; it stays split for the
+// order of its sums, as above.  The pick is the fastest split count at 256-3840
+// tokens but one (512 tokens: 12 splits 34.2, 8 splits 32.5); at 150 tiles three
+// splits (450 workgroups) beat two (o: 113 / 123).
 constexpr int WIDE_SPLIT_WGS = 256;
 constexpr int WIDE_MAX_SPLITS = 16;
 

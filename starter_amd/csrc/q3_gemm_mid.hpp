@@ -1,7 +1,9 @@
 // Dense BF16 projection for token counts too small for the 256 x 256 tiling:
-// decode batches above 64 rows and prompts up to a few hundred tokens.
+// decode batches above 64 rows, prompts below 256 tokens, and of longer ones
+// gate/up up to 512 tokens and q|k|v at 1281-1536, where that tiling is neither
+// full nor split.
 //
-// y[m, n] = epi(sum_k x[m, k] * W[n, k]).  At 9-512 tokens a projection moves
+// y[m, n] = epi(sum_k x[m, k] * W[n, k]).  At these sizes a projection moves
 // about as many bytes of activations through each CU as of weights, and both
 // far outweigh the arithmetic, so the kernel is built around two streams that
 // never wait for each other:
@@ -14,27 +16,30 @@
 //     loads), and two DPP moves per register make operands of two loads.  With
 //     several token tiles the weights are shared through L2 and L1: plain loads
 //     in operand order, the second instruction of a line finding it in L1;
-//     non-temporal ones fetch the line again (gate/up at 16 tokens, us:
-//     non-temporal half lines 26.3, plain half lines 20.6, whole lines 18.2; at
-//     100 tokens 35.3 / 30.7 / 27.1);
+//     non-temporal ones fetch the line again (gate/up at 16 / 45 / 100 tokens,
+//     us, one process: non-temporal half lines 30.1 / 32.5 / 37.4, plain half
+//     lines 22.0 / 25.9 / 34.2, whole lines 20.3 / 24.0 / 33.1);
 //   * the 16 * MB token rows of a step are filled into LDS by loader waves
 //     with direct global-to-LDS loads, STAGES - 1 steps ahead, and feed
 //     every compute wave as B operands.  Waves of their own, because vector
 //     memory counters retire in order: a compute wave that loaded both would
-//     wait for its newest token rows with every weight it needs.  One wave
-//     streams at most ~27 GB/s whatever its depth, four ~100 GB/s, hence the
-//     loader counts (gate/up at 250 tokens: two loaders 57 us, four 45).
+//     wait for its newest token rows with every weight it needs.
 // A workgroup is NW compute waves (16 NB NW weight rows) and the loader waves,
 // one barrier per step.
 //
-// What bounds it: the weights' HBM stream (5.5 TB/s at 16 tokens on gate/up,
-// launch included) and, from ~64 tokens on, the token rows beside it: without
-// them gate/up takes 21 us at 100 tokens, without the weights 10, without MFMAs
-// or LDS reads as long as with them.  Measured
-// against the register-staged 128 x 128 tiling that it replaced (us, cold
-// weights, splits included): 45 tokens qkv 36.6 -> 10.9, o 56.7 -> 10.4,
-// gate/up 40.3 -> 20.5, down 131 -> 14; 100 tokens 47.5 -> 14.1, 73.7 ->
-// 13.7, 50.0 -> 27.1, 169 -> 18; o unsplit at 1000 tokens 76 -> 35.
+// What bounds it: the CU's memory path, which carries the weights' HBM stream
+// (5.2 TB/s at 16 tokens on gate/up, launch included) and the token rows from
+// L2 beside it.  Copies of the kernel, gate/up at 45 / 100 tokens (24.0 / 33
+// us): without the token loads 20.0 / 22.2, without the weight loads past the
+// first steps 12.8 / 19.1, without the LDS reads 24.1 / 32.9, without the MFMAs
+// 24.3 / 33.5.  Counters agree: waves wait for LDS in 0.9 / 2.5% of their
+// cycles, no bank conflicts, MFMA busy 7 / 12%.
+//
+// Against the register-staged tiles (us, cold weights; where the weights were
+// allocated moves gate/up by up to 8%): 45 tokens qkv 36.5 -> 12-13, o 56.7 ->
+// 11.3, gate/up 40.4 -> 22-24, down 129.4 -> 23.4; 100 tokens 47.6 -> 14.5, 73.5
+// -> 13.2, 50.5 -> 30-33, 169 -> 27.9; 512 tokens gate/up 93.0 -> 88.5; qkv at
+// 1400 tokens 85.5 -> 73.3.
 #pragma once
 
 #include "q3_common.hpp"
@@ -90,7 +95,8 @@ struct MidArgs {
 };
 
 // Loader waves: one per SIMD where the token rows of a step are most of the
-// bytes (an odd count of 16-row blocks does not deal out over four).
+// bytes (an odd count of 16-row blocks does not deal out over four; two instead
+// of four measure level, 47.6 us for gate/up at 235 tokens).
 template <int MB>
 constexpr int MID_LOADERS = MB > 4 ? (MB % 2 ? 2 : 4) : MB > 1 ? 2 : 1;
 
@@ -216,8 +222,8 @@ __global__ __launch_bounds__((NW + MID_LOADERS<MB>) * 64) void gemm_mid_kernel(M
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     // LDS reads run MID_LEAD operands ahead of their MFMAs; the compiler's own
-    // order waits for each right before its use (gate/up at 100 tokens 32.5 ->
-    // 30.7 us).
+    // order waits for each right before its use (gate/up at 235 tokens 48.8 ->
+    // 47.6 us; level at 128 and below).
     constexpr int LEAD = MB < MID_LEAD ? MB : MID_LEAD;
     auto step = [&](int c, int u) {
         const char* xp = lds + (c % STAGES) * XT;
@@ -301,7 +307,13 @@ constexpr int MID_MAX_MB = 8;
 // Picks the plan of least estimated time.  A CU's bytes set it, not its
 // arithmetic, so a step costs about 20 ns per 16-row block that the workgroup
 // loads (weights or tokens) plus 100 ns of barrier and latency, once per round
-// of workgroups over the CUs.
+// of workgroups over the CUs.  Against a sweep of all shapes at 9-512 tokens on
+// the four projections the pick is the fastest or within 3% of it at 93 of 100
+// sizes, and 4-15% off at seven that it thinks need a round less than they do
+// (down at 255 / 512 tokens 47.4 / 61.3 against 43.0 / 53.4 us, o at 512 27.5
+// against 25.3, qkv at 255 23.7 against 21.9).  Fewer tokens can take longer:
+// down at 64 tokens is two tiles of 80 workgroups (29.1 us, the fastest of the
+// shapes), at 65-80 three (25.8).
 inline MidPlan mid_plan(int M, int N, int cus) {
     const int mblocks = (M + 15) / 16, nblocks = (N + 15) / 16;
     MidPlan best{1, 1, 2};
