@@ -685,11 +685,12 @@ class Engine:
                 s_d = call("q3_gemm_splits", M, H, I)
                 # Longer prompts whose last round of tiles is at most half full split
                 # those tiles along K (q3_gemm_ws); the same buffer holds either.
-                # Below 256 tokens neither does (both sizes are 0): the sums there have
-                # one order whatever the row count, hence the same tokens.
+                # Below 256 tokens neither does (both sizes are 0, and are not asked for):
+                # the sums there have one order whatever the row count.
                 floats = max(s_o, s_d) * M * H
-                for n_, k_ in ((self.qkv_size, H), (2 * I, H), (H, self.q_size), (H, I)):
-                    floats = max(floats, call("q3_gemm_ws_floats", M, n_, k_))
+                if M >= 256:
+                    for n_, k_ in ((self.qkv_size, H), (2 * I, H), (H, self.q_size), (H, I)):
+                        floats = max(floats, call("q3_gemm_ws_floats", M, n_, k_))
                 part = _ptr(self._prefill_partials(floats)) if floats else None
                 for i, L in enumerate(self.layers):
                     if i == 0:
