@@ -46,6 +46,8 @@
 // consecutive output columns of one token row (both halves of a SwiGLU pair in
 // one lane); the wide tiling regroups them across lanes for 16-byte stores
 // where the output rows allow it (store_row16).
+#include <atomic>
+
 #include "q3_common.hpp"
 #include "q3_dma.hpp"
 #include "q3_gemm_mid.hpp"
@@ -522,15 +524,17 @@ int launch_wide(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, int K, 
 // Compute units of the current device (cached per device; 0 if unknown).
 static int cu_count() {
     constexpr int MAX_DEV = 64;
-    static int cached[MAX_DEV];  // 0 = not yet asked; -1 = unknown
+    static std::atomic<int> cached[MAX_DEV];  // 0 = not yet asked; -1 = unknown
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEV) return 0;
-    if (cached[dev] == 0) {
+    int known = cached[dev].load(std::memory_order_relaxed);
+    if (known == 0) {
         int cus = 0;
         const bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
-        cached[dev] = ok && cus > 0 ? cus : -1;
+        known = ok && cus > 0 ? cus : -1;
+        cached[dev].store(known, std::memory_order_relaxed);
     }
-    return cached[dev] > 0 ? cached[dev] : 0;
+    return known > 0 ? known : 0;
 }
 
 // The wide tiling once it has at least this many 256 x 256 tiles (with fewer,
@@ -590,8 +594,9 @@ extern "C" int q3_gemm(const bf16_t* x, int ldx, const bf16_t* w, int M, int N, 
     if (q3_gemm_tiles_wide(M, N))
         return launch_wide(x, ldx, w, M, N, K, epi, y, ldy, ((M + 255) / 256) * ((N + 255) / 256), 1, nullptr,
                            stream);
-    const MidPlan plan = mid_plan(M, N, mid_cus());
-    if (narrow_faster(plan, M, N, K, mid_cus())) return launch_narrow(x, ldx, w, M, N, K, epi, y, ldy, stream);
+    const int cus = mid_cus();
+    const MidPlan plan = mid_plan(M, N, cus);
+    if (narrow_faster(plan, M, N, K, cus)) return launch_narrow(x, ldx, w, M, N, K, epi, y, ldy, stream);
     return launch_mid(plan, x, ldx, w, M, N, K, epi, y, ldy, stream);
 }
 
